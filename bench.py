@@ -528,7 +528,10 @@ def main():
     ms_per_step = wall * 1e3 / args.steps
     value = args.nsample * args.steps / wall
 
-    # Roofline of the dominant kernel (multi-unit step).  A launch here is
+    # Roofline of the dominant kernel (multi-unit step, or with the automatic
+    # launch shape, variant -1, the resident steps: fields on the chip, a
+    # "launch" then being one step of every unit and the bytes those a step
+    # through memory would move).  A launch here is
     # one macro step of every unit: `lanes` concurrent dispatches, each over
     # its share of the units, on the lanes' streams.  Algorithmic bytes of
     # one launch / its average time, the timed region's time (events on the
@@ -573,9 +576,9 @@ def main():
                    "nsample": args.nsample, "shots": p.ns, "nt": p.nt, "grid": [p.nz, p.nx],
                    "ckpt_interval": args.ckpt, "tile_variant": variant, "launch_grid": grid,
                    "steps_per_launch": tb, "graph_steps": graph_steps, "lanes": lanes},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "hbm" if variant >= 0 else "valu", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "step_multi_kernel", "bytes_per_launch": int(bytes_per_launch),
+                     "kernel": "step_multi_kernel" if variant >= 0 else "resident_kernel", "bytes_per_launch": int(bytes_per_launch),
                      "launches_per_step": launches, "avg_launch_us": round(avg_launch_s * 1e6, 3),
                      "dispatches_per_launch": lanes, **({"profile_on_record": profile} if profile else {})},
     }

@@ -1,6 +1,8 @@
 """Launch-shape autotuner of the batched FWI-2D step.
 
-The multi-unit step has three launch knobs (process-wide, set through the C
+By default the library keeps the fields on the chip where its plan says that
+this is faster (the automatic choice, AUTOMATIC below).  The per-step kernels
+it otherwise launches have three knobs (process-wide, set through the C
 ABI): the strip-segment height (tile variant: rows per wavefront work item),
 the grid (0 = one wavefront per work item) and the time steps per launch
 (1 or 2).  Which combination is fastest depends on the grid size, the number
@@ -27,6 +29,7 @@ from .forward.fwi2d.params import FWIParams
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "geopvi_amd", "autotune.json")
 
 Candidate = Tuple[int, int, int]  # (variant, grid, steps per launch)
+AUTOMATIC: Candidate = (-1, 0, 1)  # the library's own choice
 
 _lock = threading.Lock()
 
@@ -144,7 +147,8 @@ def autotune(params: FWIParams, nsample: int, cands: Optional[Sequence[Candidate
 
     Returns {"variant", "grid", "tb", "us_per_step", "cached", "timings"}.
     With a cache path, a previous result for the same device and shape is
-    applied without measuring (unless `force`)."""
+    applied without measuring (unless `force`, or it was measured without the
+    automatic choice among the default candidates)."""
     if device_name is None:
         if timer is not None:
             device_name = "test"
@@ -154,12 +158,15 @@ def autotune(params: FWIParams, nsample: int, cands: Optional[Sequence[Candidate
     key = shape_key(params, nsample, device_name) + f"|{schedule}"
     if cache_path and not force:
         hit = load_cache(cache_path).get(key)
-        if hit and all(k in hit for k in ("variant", "grid", "tb")):
+        whole = cands is not None or timer is not None or "%d,%d,%d" % AUTOMATIC in (hit or {}).get("timings", {})
+        if hit and whole and all(k in hit for k in ("variant", "grid", "tb")):
             cand = (int(hit["variant"]), int(hit["grid"]), int(hit["tb"]))
             if timer is None:
                 apply(cand)
             return {**hit, "cached": True}
-    cands = list(cands) if cands is not None else candidates()
+    if cands is None:
+        cands = candidates() + ([AUTOMATIC] if timer is None else [])
+    cands = list(cands)
     timings = measure(params, nsample, cands, steps=steps, device=device, timer=timer, schedule=schedule)
     best = select(timings)
     if timer is None:

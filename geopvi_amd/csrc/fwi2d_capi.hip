@@ -326,11 +326,90 @@ Sched make_sched(const Geom& g, int ckpt_req)
     return s;
 }
 
+// ---------------------------------------------------------------------------
+// Resident steps (fwi2d_resident.hip): the slabs of a unit.  More slabs mean
+// shorter steps and more exchanges; a launch runs cus / slabs units at a time.
+// The time of a step of all units is modelled as rounds x (fixed + cost of the
+// busiest SIMD); the plan of least time is kept per geometry and unit count.
+//
+// Whether the batch takes it: the modelled time of a resident step against that
+// of a per-step launch (microseconds, fitted to forward + adjoint runs of 34
+// batches; the resident side 6 % high, so that a near tie keeps the launches).
+// The fields of a wide grid fill the LDS with a few rows per slab, whose halo
+// rows then cost more than their own.  Measured, resident and per-step launch,
+// us a step: 2 units of 52x68 padded points 5.0 and 13.1, 64 of 148x228 7.6 and
+// 16.6, 20 of 228x428 8.2 and 15.5, 320 of them 86 and 124; 30 of 228x728 20
+// and 29, 80 of them 54 and 51; 16 of 328x928 26 and 27, 30 of them 49 and 36.
+constexpr double kResRoundUs = 1.06, kResRowUs = 0.072, kResHaloRows = 2.2;
+constexpr double kStepUs = 12.0, kStepUsPerMpoint = 3.0, kStepUsPerLc = 0.09;
+constexpr int kResCus = 256;
+constexpr int kResTickets = 4096;    // launches between two clears
+constexpr int kResChunk = 256;       // time steps per launch
+
+struct ResChoice {
+    bool ok;
+    ResPlan plan;
+};
+std::mutex g_res_mu;
+std::map<std::tuple<int, int, int, int, int>, ResChoice> g_res_plans;
+constexpr size_t kMaxResPlans = 256;
+
+void res_choose(const Geom& g, int units, ResChoice* out)
+{
+    out->ok = false;
+    if (g.lc == 0) return;
+    const auto key = std::make_tuple(g.ntx, g.ntz, g.lc, g.pml, units);
+    std::lock_guard<std::mutex> lk(g_res_mu);
+    auto it = g_res_plans.find(key);
+    if (it != g_res_plans.end()) {
+        *out = it->second;
+        return;
+    }
+    // Slab counts in the order of a lower bound on their time (equal work on
+    // every SIMD); the search ends where the bound passes the best plan found.
+    const ResGeom rg{g.ntx, g.ntz, g.lc, g.pml};
+    const double work = res_work(rg) / 4;
+    auto rounds = [&](int slabs) {
+        const int at_once = std::max(1, kResCus / slabs);
+        return (double)((units + at_once - 1) / at_once);
+    };
+    auto bound = [&](int slabs) { return rounds(slabs) * (res_fixed(rg, slabs) + work / slabs); };
+    int order[kResMaxSlabs];
+    for (int i = 0; i < kResMaxSlabs; ++i) order[i] = i + 1;
+    std::stable_sort(order, order + kResMaxSlabs, [&](int a, int b) { return bound(a) < bound(b); });
+    double best = 1e300;
+    for (int slabs : order) {
+        if (bound(slabs) >= best) break;
+        ResPlan p;
+        const double c = res_make_plan(rg, slabs, &p, best / rounds(slabs) - res_fixed(rg, slabs));
+        if (c < 0) continue;
+        best = rounds(slabs) * (res_fixed(rg, slabs) + c);
+        out->ok = true;
+        out->plan = p;
+    }
+    if (out->ok) {
+        const int n = out->plan.slabs;
+        const double halo = n > 1 ? kResHaloRows * 2 * out->plan.hr * g.ntx / 256.0 : 0.0;
+        const double res_us = rounds(n) * (kResRoundUs + kResRowUs * halo) + kResRowUs * best;
+        const double step_us = kStepUs + kStepUsPerMpoint * (1 + kStepUsPerLc * (g.lc - 4)) * 1e-6 * units * g.ntx * g.ntz;
+        out->ok = res_us < step_us;
+    }
+    if (g_res_plans.size() >= kMaxResPlans) g_res_plans.clear();
+    g_res_plans[key] = *out;
+}
+
+int64_t res_halo_words(const Geom& g, const ResPlan& p)
+{
+    return (int64_t)(p.slabs - 1) * 2 * 2 * p.hr * g.ntx;
+}
+
 // Field-buffer pointers of the layouts below point at row 0 (origin) of
 // their first buffer.
 struct BatchLayout {
     float *vel, *wav, *fwd, *adj, *ck, *save, *gpriv, *zero;
     double* partial;
+    unsigned long long* halo;   // resident steps: words sent between slabs, per unit, then kResTickets ticket counters
+    int64_t halo_stride, vel_stride;   // vel_stride: fe, or 2 fe with (v dt)^2 behind each sample's velocities
     double* fft;    // pseudo-spectral path: per unit, ntz rows of 2 (ntx/2 + 1) doubles (in-place r2c/c2r)
     float* ktab;    // pseudo-spectral path: |k|^2 per padded point
     double* twid;   // pseudo-spectral path: (cos, sin)(2 pi m / n), m < n, for n = ntx, then for n = ntz
@@ -355,7 +434,17 @@ void batch_layout(const Geom& g, const Sched& sc, int nsample, bool tables, char
     L->save_stride = model_only ? 0 : rnd((int64_t)sc.nslot * g.ni);
     L->grad_stride = model_only ? 0 : rnd(g.ni);
     auto org = [&](float* p) { return p ? p + g.origin : nullptr; };
-    L->vel = org(b.take<float>((size_t)nsample * g.fe));
+    ResChoice rc;
+    rc.ok = false;
+    if (tables) res_choose(g, (int)U, &rc);
+    L->vel_stride = rc.ok ? 2 * g.fe : g.fe;
+    L->vel = org(b.take<float>((size_t)(nsample * L->vel_stride)));
+    L->halo = nullptr;
+    L->halo_stride = 0;
+    if (rc.ok) {
+        L->halo_stride = res_halo_words(g, rc.plan);
+        L->halo = b.take<unsigned long long>((size_t)(U * L->halo_stride) + kResTickets / 2);
+    }
     L->zero = org(b.take<float>((size_t)g.fe));
     L->wav = b.take<float>(g.nt + g.pml0 + 1);  // wavelet, then the ABC taper table
     L->fwd = org(b.take<float>((size_t)(U * L->fwd_stride)));
@@ -423,6 +512,7 @@ JobDesc make_job(const gpvi_fwi2d_params* p, const Geom& g, const Sched& sc, int
     for (int c = 0; c < 8; ++c) j.fd[c] = g.fd[c];
     j.fe = g.fe;
     j.wtab = L.wav + g.nt;
+    j.vel_stride = L.vel_stride;
     j.fwd_stride = L.fwd_stride; j.adj_stride = L.adj_stride; j.ck_stride = L.ck_stride;
     j.save_stride = L.save_stride; j.grad_stride = L.grad_stride;
     j.fwd = L.fwd; j.adj = L.adj; j.ck = L.ck; j.save = L.save; j.gpriv = L.gpriv;
@@ -432,9 +522,9 @@ JobDesc make_job(const gpvi_fwi2d_params* p, const Geom& g, const Sched& sc, int
 
 // Per-job device set-up: padded models, wavelet and taper, the zero field.
 int job_setup(hipStream_t st, const gpvi_fwi2d_params* p, const Geom& g, const float* vel_inner, float* vel,
-              float* wav, float* zero, int nsample)
+              int64_t vel_stride, float* wav, float* zero, int nsample)
 {
-    HIP_TRY(launch_pad_velocity(st, vel_inner, vel, g.nx, g.nz, g.pml, g.ntx, g.ntz, g.pitch, g.fe, nsample));
+    HIP_TRY(launch_pad_velocity(st, vel_inner, vel, g.nx, g.nz, g.pml, g.ntx, g.ntz, g.pitch, vel_stride, nsample));
     HIP_TRY(launch_tables(st, wav, g.nt, p->dt, p->f0, wav + g.nt, g.pml0));
     HIP_TRY(launch_zero(st, zero - g.origin, g.fe));
     return 0;
@@ -456,6 +546,33 @@ int step_capacity(int lc, int tb)
     if (cap < 8) cap = 2048;  // occupancy query unavailable: 8 waves per SIMD on 256 CUs
     cache[key] = cap;
     return cap;
+}
+
+// The same for the resident kernels (0: not available on this device).
+int res_capacity(int lc)
+{
+    static std::mutex mu;
+    static std::map<std::pair<int, int>, int> cache;
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const auto key = std::make_pair(dev, lc);
+    std::lock_guard<std::mutex> lk(mu);
+    auto it = cache.find(key);
+    if (it != cache.end()) return it->second;
+    return cache[key] = resident_capacity(lc);
+}
+
+// CUs that work on this stream may use (a stream can be made with a CU mask).
+int stream_cus(hipStream_t st)
+{
+    uint32_t mask[32] = {0};
+    if (hipExtStreamGetCUMask(st, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1 << 30;
+    }
+    int n = 0;
+    for (uint32_t m : mask) n += __builtin_popcount(m);
+    return n ? n : 1 << 30;
 }
 
 // Workgroups of one multi-unit launch (a multiple of 8): the tuned grid if
@@ -811,7 +928,7 @@ static int plain_run(const gpvi_fwi2d_params* p, const float* vel_inner, float* 
     if ((rc = check_workspace(workspace, workspace_bytes, L.bytes))) return rc;
     plain_layout(g, (char*)workspace, adjoint, &L);
     hipStream_t st = (hipStream_t)stream;
-    if ((rc = job_setup(st, p, g, vel_inner, L.vel, L.wav, L.zero, 1))) return rc;
+    if ((rc = job_setup(st, p, g, vel_inner, L.vel, g.fe, L.wav, L.zero, 1))) return rc;
     UnitDesc u = plain_unit(p, g);
     u.fwd = L.fwd; u.adj = L.adj; u.save = L.save; u.grad = grad; u.vel = L.vel; u.wav = L.wav;
     u.wtab = L.wav + g.nt;
@@ -942,7 +1059,7 @@ int psm_plans(int ntz, int ntx, int batch, hipStream_t st, PsmPlans* out)
 // between.  A later forward call on the same address replaces the stamp.
 struct LayoutStamp {
     gpvi_fwi2d_params p;
-    int nsample, ckpt, variant, tb;
+    int nsample, ckpt, variant, tb, resident;
     unsigned long long seq;
 };
 std::mutex g_stamp_mu;
@@ -950,7 +1067,7 @@ std::map<const void*, LayoutStamp> g_stamps;
 unsigned long long g_stamp_seq = 0;
 constexpr size_t kMaxStamps = 4096;
 
-void layout_stamp_put(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, const Tuning& tn)
+void layout_stamp_put(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, const Tuning& tn, bool resident)
 {
     std::lock_guard<std::mutex> lk(g_stamp_mu);
     if (g_stamps.size() >= kMaxStamps && !g_stamps.count(ws)) {
@@ -959,10 +1076,10 @@ void layout_stamp_put(const void* ws, const gpvi_fwi2d_params* p, int nsample, i
             if (it->second.seq < oldest->second.seq) oldest = it;
         g_stamps.erase(oldest);
     }
-    g_stamps[ws] = LayoutStamp{*p, nsample, ckpt, tn.variant, tn.tb, ++g_stamp_seq};
+    g_stamps[ws] = LayoutStamp{*p, nsample, ckpt, tn.variant, tn.tb, resident ? 1 : 0, ++g_stamp_seq};
 }
 
-int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, Tuning* tn)
+int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, Tuning* tn, bool* resident)
 {
     std::lock_guard<std::mutex> lk(g_stamp_mu);
     auto it = g_stamps.find(ws);
@@ -975,6 +1092,54 @@ int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, in
                                       "phase that prepared this workspace");
     tn->variant = s.variant;
     tn->tb = s.tb;
+    *resident = s.resident != 0;
+    return 0;
+}
+
+// The batch's steps with the fields on the chip: launches of up to kResChunk
+// steps, each within one pass (forward, a segment's recompute, an adjoint
+// stretch).
+int res_run(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom& g, const Sched& sc, const JobDesc& j,
+            const BatchLayout& L, const ResPlan& plan, int capacity)
+{
+    const int64_t units = (int64_t)nsample * g.ns;
+    unsigned* const tickets = reinterpret_cast<unsigned*>(L.halo + units * L.halo_stride);
+    HIP_TRY(launch_zero(st, reinterpret_cast<float*>(L.halo), 2 * units * L.halo_stride + kResTickets));
+    HIP_TRY(launch_vdt2(st, L.vel, L.vel + g.fe, p->dt, (int64_t)g.ntz * g.pitch, L.vel_stride, nsample));
+    UnitDesc sd;
+    std::memset(&sd, 0, sizeof sd);
+    sd.nt = g.nt; sd.tb = 1; sd.nseg = sc.nseg; sd.ckpt = sc.ckpt; sd.last_len = sc.last_len;
+    auto at = [&](int s) { return decode_step(sd, s + j.s_off); };
+    ResArgs a;
+    a.units = L.units;
+    a.halo = L.halo;
+    a.halo_stride = L.halo_stride;
+    a.vdt2_off = (int)(g.fe * sizeof(float));
+    a.plan = plan;
+    a.nunit = (int)units;
+    a.clusters = std::max(1, std::min((int)units, capacity / plan.slabs));
+    int used = 0;
+    for (int s = 0; s < j.total;) {
+        const StepInfo first = at(s);
+        int n = 1;
+        while (n < kResChunk && s + n < j.total) {
+            const StepInfo q = at(s + n);
+            if (q.mode != first.mode || q.seg != first.seg) {
+                // the forward pass runs through its checkpoint segments
+                if (!(q.mode == kFwd && first.mode == kFwd)) break;
+            }
+            ++n;
+        }
+        if (used == kResTickets) {
+            HIP_TRY(launch_zero(st, reinterpret_cast<float*>(tickets), kResTickets));
+            used = 0;
+        }
+        a.ticket = tickets + used++;
+        a.s0 = s + j.s_off;
+        a.n = n;
+        HIP_TRY(launch_resident(st, g.lc, first.mode == kAdj, a));
+        s += n;
+    }
     return 0;
 }
 
@@ -1055,11 +1220,13 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
         (phase != GPVI_PHASE_FORWARD && !grad))
         return fail(GPVI_ERR_INVALID, "NULL buffer");
     Tuning tn = tuning();
+    // Resident steps unless a launch shape of the per-step kernels is set.
+    bool resident = tn.variant < 0 && tn.grid == 0 && tn.tb == 1;
     // The adjoint phase continues the forward phase's workspace: it must use
     // the layout that phase used (tile variant and steps per launch fix the
     // strip width, band items, row shift, pitch and field stride), whatever
     // the process-wide tuning says now.
-    rc = phase == GPVI_PHASE_ADJOINT ? layout_stamp_get(workspace, p, nsample, ckpt_interval, &tn)
+    rc = phase == GPVI_PHASE_ADJOINT ? layout_stamp_get(workspace, p, nsample, ckpt_interval, &tn, &resident)
                                      : 0;
     if (rc) return rc;
     if (tn.variant < 0) tn.variant = auto_variant(p, nsample, tn);
@@ -1075,9 +1242,14 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     batch_layout(g, sc, nsample, true, (char*)workspace, &L, model_only);
     hipStream_t st = (hipStream_t)stream;
     if (phase != GPVI_PHASE_ADJOINT) {
-        if ((rc = job_setup(st, p, g, vel_inner, L.vel, L.wav, L.zero, nsample))) return rc;
+        if ((rc = job_setup(st, p, g, vel_inner, L.vel, L.vel_stride, L.wav, L.zero, nsample))) return rc;
     }
-    if (phase == GPVI_PHASE_FORWARD && !model_only) layout_stamp_put(workspace, p, nsample, ckpt_interval, tn);
+    ResChoice rcho;
+    res_choose(g, nsample * g.ns, &rcho);
+    const int res_cap = resident && rcho.ok && L.halo ? std::min(res_capacity(g.lc), stream_cus(st)) : 0;
+    resident = res_cap > 0 && res_cap >= rcho.plan.slabs;
+    if (phase == GPVI_PHASE_FORWARD && !model_only)
+        layout_stamp_put(workspace, p, nsample, ckpt_interval, tn, resident);
     const int store = (phase == GPVI_PHASE_FORWARD && (flags & GPVI_FLAG_NO_STORE)) ? 0 : 1;
     JobDesc j = make_job(p, g, sc, nsample, L, record_obs, record_syn, run_fwi, phase, store);
     // Lanes: the units split into groups with contiguous runs of the tile
@@ -1087,7 +1259,7 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     int nlane = 1;
     int lane_t0[kMaxLanes] = {0}, lane_n[kMaxLanes] = {nsample * g.ns * per_unit};
     hipStream_t lane_st[kMaxLanes] = {st};
-    if (tn.lanes > 1 && !(flags & GPVI_FLAG_ONE_STREAM) && nsample * g.ns >= 2) {
+    if (!resident && tn.lanes > 1 && !(flags & GPVI_FLAG_ONE_STREAM) && nsample * g.ns >= 2) {
         const int want = nsample >= 2 ? std::min(tn.lanes, nsample) : 2;
         int have = 1;
         while (have < want) {
@@ -1135,6 +1307,14 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
         if (phase != GPVI_PHASE_ADJOINT && misfit)
             HIP_TRY(launch_misfit(st, record_syn, record_obs, (int64_t)g.ns * g.nt * g.nr, nsample, L.partial,
                                   misfit));
+        return 0;
+    }
+    if (resident) {
+        if ((rc = res_run(st, p, nsample, g, sc, j, L, rcho.plan, res_cap))) return rc;
+        if (phase != GPVI_PHASE_FORWARD)
+            HIP_TRY(launch_grad_reduce(st, L.gpriv, L.grad_stride, grad, g.ns, g.ni, nsample));
+        if (phase != GPVI_PHASE_ADJOINT && misfit)
+            HIP_TRY(launch_misfit(st, record_syn, record_obs, (int64_t)g.ns * g.nt * g.nr, nsample, L.partial, misfit));
         return 0;
     }
     int grid[kMaxLanes];
@@ -1439,7 +1619,7 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
         engine_free_slots(e, first, jb.nunit);
         return fail(GPVI_ERR_HIP, "hipEventCreate: %s", hipGetErrorString(err));
     }
-    if ((rc = job_setup(e->stream, p, jb.g, vel_inner, jb.L.vel, jb.L.wav, jb.L.zero, nsample))) {
+    if ((rc = job_setup(e->stream, p, jb.g, vel_inner, jb.L.vel, jb.L.vel_stride, jb.L.wav, jb.L.zero, nsample))) {
         engine_free_slots(e, first, jb.nunit);
         (void)hipEventDestroy(jb.done);
         return rc;

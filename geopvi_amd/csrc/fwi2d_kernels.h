@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "fwi2d_device.h"
+#include "fwi2d_resident.h"
 
 namespace gpvi {
 
@@ -30,7 +31,7 @@ struct JobDesc {
     float fd[8];
     int64_t fe;
     const float* wtab;
-    int64_t fwd_stride, adj_stride, ck_stride, save_stride, grad_stride;
+    int64_t vel_stride, fwd_stride, adj_stride, ck_stride, save_stride, grad_stride;
     float* fwd;
     float* adj;
     float* ck;
@@ -65,6 +66,22 @@ hipError_t launch_build_units(hipStream_t st, const JobDesc& j, UnitDesc* units,
 hipError_t launch_grad_reduce(hipStream_t st, const float* gpriv, int64_t grad_stride, float* out, int ns,
                               int ni, int nsample);
 int misfit_blocks(int64_t len);
+
+// Resident steps (fwi2d_resident.hip): `n` macro steps of one pass from macro
+// step s0 for every unit of the table, fields on the chip.
+struct ResArgs {
+    const UnitDesc* units;
+    unsigned long long* halo;   // halo_stride words per unit, zero before the call's first launch
+    unsigned* ticket;           // zero before every launch
+    int64_t halo_stride;
+    int vdt2_off;               // bytes from a sample's padded velocities to its (v dt)^2
+    int s0, n;
+    int nunit, clusters;        // units of the table; groups of plan.slabs workgroups
+    ResPlan plan;
+};
+hipError_t launch_resident(hipStream_t st, int lc, bool adjoint, const ResArgs& a);
+hipError_t launch_vdt2(hipStream_t st, const float* vel, float* out, float dt, int64_t n, int64_t stride, int nsample);
+int resident_capacity(int lc);
 
 // Pseudo-spectral Laplacian path (fwi2d_psm.hip).
 hipError_t launch_psm_wavenumber(hipStream_t st, float* k, int ntx, int ntz, float dx, float dz);

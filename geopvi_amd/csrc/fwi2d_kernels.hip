@@ -81,7 +81,7 @@ __global__ void ctl_set_kernel(StepCtl* ctl, int step, int n4, int n5, int n6, i
 // Edge-replicated padding of nsample inner models (fdtd2D_modelling.c:1187-1238):
 // padded(iz, ix) = inner(clamp(iz - pml), clamp(ix - pml)).
 __global__ void pad_velocity_kernel(const float* __restrict__ vin, float* __restrict__ vpad, int nx,
-                                    int nz, int pml, int ntx, int ntz, int pitch, int64_t fe, int nsample)
+                                    int nz, int pml, int ntx, int ntz, int pitch, int64_t stride, int nsample)
 {
     const int64_t per = (int64_t)ntz * pitch;
     const int64_t total = per * nsample;
@@ -96,7 +96,7 @@ __global__ void pad_velocity_kernel(const float* __restrict__ vin, float* __rest
             const int jx = min(max(ix - pml, 0), nx - 1);
             val = vin[(int64_t)m * nx * nz + (int64_t)jz * nx + jx];
         }
-        vpad[(int64_t)m * fe + r] = val;
+        vpad[(int64_t)m * stride + r] = val;
     }
 }
 
@@ -179,7 +179,7 @@ __global__ void build_units_kernel(JobDesc j, UnitDesc* __restrict__ units, Tile
     u.ck = j.ck ? j.ck + (int64_t)un * j.ck_stride : nullptr;
     u.save = j.save + (int64_t)un * j.save_stride;
     u.grad = j.gpriv + (int64_t)un * j.grad_stride;
-    u.vel = j.vel + (int64_t)m * j.fe;
+    u.vel = j.vel + (int64_t)m * j.vel_stride;
     u.zero = j.zero;
     u.wav = j.wav;
     u.syn = j.syn + ((int64_t)m * j.ns + sh) * j.nt * j.nr;
