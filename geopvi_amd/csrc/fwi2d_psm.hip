@@ -94,23 +94,38 @@ __global__ void psm_scale_kernel(double2* __restrict__ spec, const float* __rest
     }
 }
 
-// p1, p0 and v at point (iz, ix) of a unit.
+// What the update of point (iz, ix) of a unit reads: p1, p0 and v, and in
+// the absorbing bands the taper weight, p1 two cells and p0 four cells inward
+// along z and along x (the two edges of an axis do not overlap).
 struct PsmCore {
     float p1, p0, v;
+    float z[7], x[7];   // weight, p1 at 1, 2 and p0 at 1..4 cells inward
 };
 __device__ inline unsigned psm_vo(const PointConsts& kc, int iz, int ix, int ro)
 {
     return (unsigned)((iz + kPadRows) * kc.pitch4 + ix * 4 - ro);
 }
+__device__ inline void psm_band(float* b, Rsrc w, int cell, Rsrc p1, Rsrc p0, unsigned vo, int step)
+{
+    b[0] = bload(w, (unsigned)cell * 4u, 0);
+#pragma unroll
+    for (int i = 1; i <= 2; ++i) b[i] = bload(p1, vo + (unsigned)(i * step), 0);
+#pragma unroll
+    for (int i = 1; i <= 4; ++i) b[i + 2] = bload(p0, vo + (unsigned)(i * step), 0);
+}
 __device__ inline PsmCore psm_core(const UnitDesc& u, const FieldPtrs& f, const PointConsts& kc, int iz, int ix)
 {
     const int64_t margin = (int64_t)kPadRows * u.pitch;
-    const int ro = 4 * kc.pitch4 + 16;
-    const unsigned vo = psm_vo(kc, iz, ix, ro);
+    const unsigned vo = psm_vo(kc, iz, ix, 0);
+    const Rsrc rp1 = make_rsrc(f.p1 - margin), rp0 = make_rsrc(f.p0 - margin), rw = make_rsrc(u.wtab);
     PsmCore r;
-    r.p1 = bload(make_rsrc(f.p1 - margin), vo, ro);
-    r.p0 = bload(make_rsrc(f.p0 - margin), vo, ro);
-    r.v = bload(make_rsrc(u.vel - margin), vo, ro);
+    r.p1 = bload(rp1, vo, 0);
+    r.p0 = bload(rp0, vo, 0);
+    r.v = bload(make_rsrc(u.vel - margin), vo, 0);
+    const int dz = iz < kc.pml ? 1 : iz >= kc.ntz - kc.pml ? -1 : 0;
+    const int dx = ix < kc.pml ? 1 : ix >= kc.ntx - kc.pml ? -1 : 0;
+    if (dz) psm_band(r.z, rw, dz > 0 ? iz : kc.ntz - iz - 1, rp1, rp0, vo, dz * kc.pitch4);
+    if (dx) psm_band(r.x, rw, dx > 0 ? ix : kc.ntx - ix - 1, rp1, rp0, vo, dx * 4);
     return r;
 }
 
@@ -122,40 +137,23 @@ __device__ inline float psm_point(const UnitDesc& u, const FieldPtrs& f, const S
                                   int iz, int ix, double re, double div, PsmCore core)
 {
     const int ntx = kc.ntx, ntz = kc.ntz, pml = kc.pml, pitch4 = kc.pitch4;
-    const int64_t margin = (int64_t)kPadRows * u.pitch;
-    // byte offset of (iz, ix) from the first margin row, split so that the
-    // inward reads (up to 4 rows or columns either way) stay >= 0
     const int ro = 4 * pitch4 + 16;
     const unsigned vo = psm_vo(kc, iz, ix, ro);
-    const Rsrc rp1 = make_rsrc(f.p1 - margin);
-    const Rsrc rp0 = make_rsrc(f.p0 - margin);
     const float p1c = core.p1, p0c = core.p0, v = core.v;
     const float vdt = v * kc.dt;
     float val = (float)((double)(2.f * p1c - p0c) + (double)(vdt * vdt) * re / div);
 
-    const bool top = iz < pml, bot = iz >= ntz - pml, lef = ix < pml, rig = ix >= ntx - pml;
-    if (top || bot || lef || rig) {
+    const bool zb = iz < pml || iz >= ntz - pml, xb = ix < pml || ix >= ntx - pml;
+    if (zb || xb) {
         const float sc = div1_const(v * kc.dt, kc.dx, kc.rdx, kc.hi, kc.ydx);
         const float t11 = ((2.f - sc) * (1.f - sc)) / 2.f;
         const float t12 = sc * (2.f - sc);
         const float t13 = (sc * (sc - 1.f)) / 2.f;
-        const Rsrc rw = make_rsrc(u.wtab);
-        if (top)
-            val = abc_blend(bload(rw, (unsigned)iz * 4u, 0),
-                            abc_extrapolate(p1c, bload(rp1, vo, ro + pitch4), bload(rp1, vo, ro + 2 * pitch4), rp0,
-                                            vo, ro, pitch4, t11, t12, t13), val);
-        if (bot)
-            val = abc_blend(bload(rw, (unsigned)(ntz - iz - 1) * 4u, 0),
-                            abc_extrapolate(p1c, bload(rp1, vo, ro - pitch4), bload(rp1, vo, ro - 2 * pitch4), rp0,
-                                            vo, ro, -pitch4, t11, t12, t13), val);
-        if (lef)
-            val = abc_blend(bload(rw, (unsigned)ix * 4u, 0),
-                            abc_extrapolate(p1c, bload(rp1, vo, ro + 4), bload(rp1, vo, ro + 8), rp0, vo, ro, 4, t11,
-                                            t12, t13), val);
-        if (rig)
-            val = abc_blend(bload(rw, (unsigned)(ntx - ix - 1) * 4u, 0),
-                            abc_extrapolate(p1c, bload(rp1, vo, ro - 4), bload(rp1, vo, ro - 8), rp0, vo, ro, -4, t11,
-                                            t12, t13), val);
+        auto blend = [&](const float* b) {
+            val = abc_blend(b[0], abc_extrap(p1c, b[1], b[2], p0c, b[3], b[4], b[5], b[6], t11, t12, t13), val);
+        };
+        if (zb) blend(core.z);
+        if (xb) blend(core.x);
     }
     const float dt = kc.dt;
     const bool rec_row = iz == u.r_iz;
@@ -227,19 +225,27 @@ __global__ void psm_twiddle_kernel(Cx* __restrict__ tw, int ntx, int ntz)
 
 __device__ inline void psm_table(Cx* T, const Cx* __restrict__ tw, int n)
 {
-    for (int m = threadIdx.x; m < spec::table_len(n); m += blockDim.x) T[m] = tw[m];
+    for (int m = threadIdx.x; m < spec::table_len(n); m += spec::kThreads) T[m] = tw[m];
 }
 
 // The plan's passes over nseq sequences, x -> y -> x ... (a barrier after
 // each); returns the buffer holding the result.  Expects a barrier before.
+// tw: the whole table in memory, from which the odd radices' roots, the same
+// for every thread, are scalar loads.
+#ifdef __HIP_DEVICE_COMPILE__
+typedef const __attribute__((address_space(4))) double* RootPtr;
+#else
+typedef const double* RootPtr;
+#endif
 template <int MaxR>
-__device__ inline Cx* psm_transform(Cx* x, Cx* y, int nseq, const spec::Plan& p, const Cx* T, int sgn)
+__device__ inline Cx* psm_transform(Cx* x, Cx* y, int nseq, const spec::Plan& p, const Cx* T, const Cx* tw, int sgn)
 {
-    int ns = 1;
+    const RootPtr roots = (RootPtr)(uint64_t)tw;
     for (int i = 0; i < p.npass; ++i) {
-        spec::run_pass<MaxR>(p.radix[i], x, y, nseq, p.n, ns, T, sgn, threadIdx.x, blockDim.x);
+        spec::run_pass<MaxR>(
+            p.pass[i], x, y, nseq, p.n, T,
+            [&](int m) { return spec::cx(roots[2 * m], roots[2 * m + 1]); }, sgn, threadIdx.x, spec::kThreads);
         __syncthreads();
-        ns *= p.radix[i];
         Cx* t = x;
         x = y;
         y = t;
@@ -266,12 +272,12 @@ psm_rows_fwd_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ 
     psm_table(T, tw, ntx);
     const float* p1 = f.p1;
     const int pitch = u.pitch;
-    spec::rows_load(X, np, ntx, ntz, pair0, [&](int iz, int ix) { return (double)p1[(int64_t)iz * pitch + ix]; },
-                    threadIdx.x, blockDim.x);
+    spec::rows_load(X, np, ntx, ntz, pair0, [&](int iz, int ix) { return (double)p1[iz * pitch + ix]; },
+                    threadIdx.x, spec::kThreads);
     __syncthreads();
-    const Cx* Z = psm_transform<MaxR>(X, Y, np, px, T, +1);
-    spec::rows_unpack(Z, np, ntx, ntz, nc, pair0, [&](int iz, int fq, Cx v) { sp[(int64_t)iz * nc + fq] = v; },
-                      threadIdx.x, blockDim.x);
+    const Cx* Z = psm_transform<MaxR>(X, Y, np, px, T, tw, +1);
+    spec::rows_unpack(Z, np, ntx, ntz, nc, pair0, [&](int iz, int fq, Cx v) { sp[iz * nc + fq] = v; },
+                      threadIdx.x, spec::kThreads);
 }
 
 // Columns: block (g, unit) transforms spectrum columns [g ncol, (g + 1) ncol),
@@ -298,16 +304,16 @@ psm_cols_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ spec
     Cx* X = T + spec::table_len(ntz);
     Cx* Y = X + ncol * ntz;
     psm_table(T, tw + ntx, ntz);
-    spec::cols_load(X, ncol, ntz, nc, f0, [&](int iz, int fq) { return sp[(int64_t)iz * nc + fq]; }, threadIdx.x,
-                    blockDim.x);
+    spec::cols_load(X, ncol, ntz, nc, f0, [&](int iz, int fq) { return sp[iz * nc + fq]; }, threadIdx.x,
+                    spec::kThreads);
     __syncthreads();
-    Cx* Z = psm_transform<MaxR>(X, Y, ncol, pz, T, +1);
-    spec::cols_scale(Z, ncol, ntz, nc, f0, [&](int iz, int fq) { return k[(int64_t)iz * ntx + fq]; }, threadIdx.x,
-                     blockDim.x);
+    Cx* Z = psm_transform<MaxR>(X, Y, ncol, pz, T, tw + ntx, +1);
+    spec::cols_scale(Z, ncol, ntz, nc, f0, [&](int iz, int fq) { return k[iz * ntx + fq]; }, threadIdx.x,
+                     spec::kThreads);
     __syncthreads();
-    const Cx* W = psm_transform<MaxR>(Z, Z == X ? Y : X, ncol, pz, T, -1);
-    spec::cols_store(W, ncol, ntz, nc, f0, [&](int iz, int fq, Cx v) { sp[(int64_t)iz * nc + fq] = v; },
-                     threadIdx.x, blockDim.x);
+    const Cx* W = psm_transform<MaxR>(Z, Z == X ? Y : X, ncol, pz, T, tw + ntx, -1);
+    spec::cols_store(W, ncol, ntz, nc, f0, [&](int iz, int fq, Cx v) { sp[iz * nc + fq] = v; },
+                     threadIdx.x, spec::kThreads);
 }
 
 // Rows backward and the point update: block (g, unit) transforms row pairs
@@ -330,51 +336,40 @@ psm_rows_inv_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ 
     Cx* X = T + spec::table_len(ntx);
     Cx* Y = X + np * ntx;
     psm_table(T, tw, ntx);
-    spec::rows_repack(X, np, ntx, ntz, pair0, [&](int iz, int fq) { return sp[(int64_t)iz * nc + fq]; },
-                      threadIdx.x, blockDim.x);
+    spec::rows_repack(X, np, ntx, ntz, pair0, [&](int iz, int fq) { return sp[iz * nc + fq]; },
+                      threadIdx.x, spec::kThreads);
     __syncthreads();
-    const Cx* Z = psm_transform<MaxR>(X, Y, np, px, T, -1);
+    const Cx* Z = psm_transform<MaxR>(X, Y, np, px, T, tw, -1);
     Cx* const W = Z == X ? Y : X;   // the next step's rows (chain)
     const FieldPtrs f = step_fields(u, si);
     const int64_t margin = (int64_t)kPadRows * u.pitch;
     const StepCtx c = make_step(u, si.mode, si.it, si.seg, f.out, margin);
     const PointConsts kc = point_consts(u);
     const double ntp = (double)ntx * (double)ntz;
-    // the points of the block's rows, spec::kChunk per thread at a time with
-    // their p1, p0 and v loads in flight together
+    // The points of the block's rows, one per thread at a time: the band
+    // reads of a point are in flight together, and one point's worth keeps the
+    // kernel at 61 registers (114 us a step on 80 units of 220 x 420; two
+    // points in flight, 107 registers, 135 us; four, 151 registers, 149 us).
     const int total = 2 * np * ntx;
-    for (int t0 = threadIdx.x; t0 < total; t0 += spec::kChunk * blockDim.x) {
-        PsmCore core[spec::kChunk];
-#pragma unroll
-        for (int j = 0; j < spec::kChunk; ++j) {
-            const int t = t0 + j * blockDim.x;
-            const int q = t / (2 * ntx), r = t - q * 2 * ntx;
-            const int w = r >= ntx ? 1 : 0, ix = r - w * ntx;
-            const int iz = 2 * (pair0 + q) + w;
-            if (t < total && iz < ntz) core[j] = psm_core(u, f, kc, iz, ix);
+    const spec::Div by_pair = spec::divider(2 * ntx);
+    for (int t = threadIdx.x; t < total; t += spec::kThreads) {
+        const int q = spec::quot(t, by_pair), r = t - q * 2 * ntx;
+        const int w = r >= ntx ? 1 : 0, ix = r - w * ntx;
+        const int iz = 2 * (pair0 + q) + w;
+        double* const nxt = &W[q * ntx + ix].re + w;
+        if (iz >= ntz) {
+            if (chain) *nxt = 0.0;   // the missing row of an odd last pair
+            continue;
         }
-#pragma unroll
-        for (int j = 0; j < spec::kChunk; ++j) {
-            const int t = t0 + j * blockDim.x;
-            const int q = t / (2 * ntx), r = t - q * 2 * ntx;
-            const int w = r >= ntx ? 1 : 0, ix = r - w * ntx;
-            const int iz = 2 * (pair0 + q) + w;
-            if (t >= total) continue;
-            double* const nxt = &W[q * ntx + ix].re + w;
-            if (iz >= ntz) {
-                if (chain) *nxt = 0.0;   // the missing row of an odd last pair
-                continue;
-            }
-            const Cx z = Z[q * ntx + ix];
-            const float val = psm_point(u, f, c, kc, iz, ix, w ? z.im : z.re, ntp, core[j]);
-            if (chain) *nxt = (double)val;
-        }
+        const Cx z = Z[q * ntx + ix];
+        const float val = psm_point(u, f, c, kc, iz, ix, w ? z.im : z.re, ntp, psm_core(u, f, kc, iz, ix));
+        if (chain) *nxt = (double)val;
     }
     if (!chain) return;   // uniform over the launch
     __syncthreads();
-    const Cx* F = psm_transform<MaxR>(W, W == X ? Y : X, np, px, T, +1);
-    spec::rows_unpack(F, np, ntx, ntz, nc, pair0, [&](int iz, int fq, Cx v) { sp[(int64_t)iz * nc + fq] = v; },
-                      threadIdx.x, blockDim.x);
+    const Cx* F = psm_transform<MaxR>(W, W == X ? Y : X, np, px, T, tw, +1);
+    spec::rows_unpack(F, np, ntx, ntz, nc, pair0, [&](int iz, int fq, Cx v) { sp[iz * nc + fq] = v; },
+                      threadIdx.x, spec::kThreads);
 }
 
 hipError_t launch_psm_wavenumber(hipStream_t st, float* k, int ntx, int ntz, float dx, float dz)

@@ -61,21 +61,67 @@ GPVI_SPEC_FN Cx mul(Cx a, Cx b) { return cx(a.re * b.re - a.im * b.im, a.re * b.
 // -i * sgn * x
 GPVI_SPEC_FN Cx rot(Cx x, int sgn) { return sgn > 0 ? cx(x.im, -x.re) : cx(-x.im, x.re); }
 
+// n / d for 0 <= n < 2^22, d >= 1: n + 0.5 is exact and at least 0.5 / d away
+// from the next multiple of d, more than the two roundings move the product.
+// The index splits of every phase use it: the hardware has no integer divide,
+// and its expansion cost as many instructions as a radix-4 butterfly.
+struct Div {
+    int d;
+    float r;
+};
+GPVI_SPEC_FN Div divider(int d)
+{
+    Div v;
+    v.d = d;
+    v.r = 1.0f / (float)d;
+    return v;
+}
+GPVI_SPEC_FN int quot(int n, Div v) { return (int)(((float)n + 0.5f) * v.r); }
+
 constexpr int kMaxPass = 16;
 constexpr int kThreads = 256;        // workgroup of the transform kernels
 constexpr int kLdsCx = 4096;         // LDS budget of one workgroup, in Cx (64 KiB)
 // Row pairs and spectrum columns per workgroup, at most: on the 200 x 400
 // model with 10-point bands (220 x 420) one step of 4 samples x 20 shots took
-// 150.7 us with (2, 4), 161.1 with (2, 8), 169.1 with (1, 4), 169.3 with
-// (2, 2), 179.2 with (4, 4), 193.0 with (1, 2) (256 threads; 128 threads were
-// slower in an earlier sweep).
+// 114.4 us with (2, 4), 133.6 with (3, 4), 134.5 with (1, 4), 139.4 with
+// (2, 2); 134.7 with (4, 8) and 512 threads, 129.8 with (1, 2), 131.0 with
+// (1, 4) and 143.2 with (2, 4) and 128 threads.
+//
+// What bounds the passes: vector issue (about half of the cycles, 360 and 260
+// instructions a complex element and step in the row and column kernels) and
+// the latency of 6 to 8 LDS round trips with a barrier each, at 5 wavefronts a
+// SIMD (the two LDS buffers).  Of the instructions a quarter is double
+// arithmetic, the rest index splits and addresses, so those come from the
+// host or from scalar loads: 148 us a step before, 114 us since.
 constexpr int kMaxPairs = 2;
 constexpr int kMaxCols = 4;
 
-// The radices of a length-n transform, in pass order.
+// One pass of a length-n transform: radix, butterflies per sequence (n /
+// radix), product ns of the earlier radices, table step of its twiddles
+// (n / (ns radix)), and the divisors of its index splits.
+struct PassConsts {
+    int radix, nr, ns, tstep;
+    Div by_nr, by_ns;
+};
+inline PassConsts pass_consts(int radix, int n, int ns)
+{
+    PassConsts c;
+    c.radix = radix;
+    c.nr = n / radix;
+    c.ns = ns;
+    c.tstep = n / (ns * radix);
+    c.by_nr = divider(c.nr);
+    c.by_ns = divider(ns);
+    return c;
+}
+
+// The passes of a length-n transform, in order.  (The constants come from the
+// host: formed by every thread for its few butterflies they cost a quarter of
+// the pass.)
 struct Plan {
     int n, npass;
     int radix[kMaxPass];
+    PassConsts pass[kMaxPass];
 };
 
 // Factor n into passes of radix 4 (as many as fit), then one 2 if needed, then
@@ -99,6 +145,7 @@ inline bool make_plan(int n, Plan* p)
             m /= r;
         }
     }
+    for (int i = 0, ns = 1; i < p->npass; ns *= p->radix[i++]) p->pass[i] = pass_consts(p->radix[i], n, ns);
     return m == 1;
 }
 
@@ -177,67 +224,77 @@ GPVI_SPEC_FN void dft_store(Cx* v, const double* cs, const double* sn, int sgn, 
 
 // One Stockham pass of radix R over nseq sequences of length n stored back to
 // back (src -> dst): the butterflies b = tid, tid + nthr, ... of nseq * n / R.
-// ns = product of the radices of the earlier passes.  T: the twiddle table
-// (table_len, twiddle).  sgn = +1: the e^{-i} transform, -1: e^{+i}.
-template <int R>
-GPVI_SPEC_FN void pass(const Cx* src, Cx* dst, int nseq, int n, int ns, const Cx* T, int sgn, int tid, int nthr)
+// T: the twiddle table (table_len, twiddle); root(m): (cos, sin)(2 pi m / n)
+// for m < n / 2, the same for every thread.  sgn = +1: the e^{-i} transform,
+// -1: e^{+i}.
+template <int R, class Root>
+GPVI_SPEC_FN void pass(const Cx* src, Cx* dst, int nseq, int n, const PassConsts& c, const Cx* T, Root root, int sgn,
+                       int tid, int nthr)
 {
     constexpr int H = (R - 1) / 2;
-    const int nr = n / R;
-    const int tstep = n / (ns * R);
+    const int nr = c.nr, ns = c.ns;
     double cs[H + 1], sn[H + 1];
     cs[0] = 1.0;
     sn[0] = 0.0;
     if constexpr ((R & 1) != 0) {
 #pragma unroll
         for (int m = 1; m <= H; ++m) {
-            const Cx w = twiddle(T, m * nr, n);
+            const Cx w = root(m * nr);
             cs[m] = w.re;
             sn[m] = w.im;
         }
     }
     for (int b = tid; b < nseq * nr; b += nthr) {
-        const int q = b / nr, j = b - q * nr;
-        const Cx* s = src + q * n;
-        Cx* d = dst + q * n;
-        const int k = j % ns;
+        const int q = quot(b, c.by_nr), j = b - q * nr;
+        const Cx* s = src + q * n + j;
+        const int k = j - quot(j, c.by_ns) * ns;
         Cx v[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = s[j + r * nr];
+        for (int r = 0; r < R; ++r) v[r] = s[r * nr];
         if (k > 0) {
+            const int kt = k * c.tstep;
 #pragma unroll
             for (int r = 1; r < R; ++r) {
-                const Cx w = twiddle(T, r * k * tstep, n);
+                // r kt < r n / R: the first half of the table holds it up to r = R / 2
+                const Cx w = 2 * r <= R ? T[r * kt] : twiddle(T, r * kt, n);
                 v[r] = mul(v[r], cx(w.re, -sgn * w.im));
             }
         }
-        dft_store<R>(v, cs, sn, sgn, d + (j - k) * R + k, ns);
+        dft_store<R>(v, cs, sn, sgn, dst + q * n + (j - k) * R + k, ns);
     }
 }
 
-// The pass of radix r (one of the plan's radices, all <= MaxR: a kernel that
-// needs only the small radices is not held to the registers of the large).
-template <int MaxR>
-GPVI_SPEC_FN void run_pass(int r, const Cx* src, Cx* dst, int nseq, int n, int ns, const Cx* T, int sgn, int tid,
-                           int nthr)
+// The pass of radix c.radix (one of the plan's radices, all <= MaxR: a kernel
+// that needs only the small radices is not held to the registers of the large).
+template <int MaxR, class Root>
+GPVI_SPEC_FN void run_pass(const PassConsts& c, const Cx* src, Cx* dst, int nseq, int n, const Cx* T, Root root,
+                           int sgn, int tid, int nthr)
 {
+    const int r = c.radix;
     if (r == 4) {
-        pass<4>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+        pass<4>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
     } else if (r == 2) {
-        pass<2>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+        pass<2>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
     } else if (r == 3) {
-        pass<3>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+        pass<3>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
     } else if (r == 5) {
-        pass<5>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+        pass<5>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
     } else if (r == 7) {
-        pass<7>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+        pass<7>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
     } else if constexpr (MaxR >= 11) {
         if (r == 11) {
-            pass<11>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+            pass<11>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
         } else if constexpr (MaxR >= 13) {
-            pass<13>(src, dst, nseq, n, ns, T, sgn, tid, nthr);
+            pass<13>(src, dst, nseq, n, c, T, root, sgn, tid, nthr);
         }
     }
+}
+
+// The same, the constants formed here and the roots from T.
+template <int MaxR>
+inline void run_pass(int r, const Cx* src, Cx* dst, int nseq, int n, int ns, const Cx* T, int sgn, int tid, int nthr)
+{
+    run_pass<MaxR>(pass_consts(r, n, ns), src, dst, nseq, n, T, [&](int m) { return T[m]; }, sgn, tid, nthr);
 }
 
 // The largest radix of a plan.
@@ -248,23 +305,22 @@ inline int max_radix(const Plan& p)
     return m;
 }
 
-// for t = tid, tid + nthr, ... < n: put(t, get(t)), kChunk elements at a
+// for t = tid, tid + nthr, ... < n: put(t, get(t)), Chunk elements at a
 // time with every get of a chunk before its puts, so that a thread's global
 // loads are in flight together instead of one latency per element.
-constexpr int kChunk = 4;
-template <class Get, class Put>
+template <int Chunk = 4, class Get, class Put>
 GPVI_SPEC_FN void chunked(int n, int tid, int nthr, Get get, Put put)
 {
     using V = decltype(get(0));
-    for (int t0 = tid; t0 < n; t0 += kChunk * nthr) {
-        V v[kChunk];
+    for (int t0 = tid; t0 < n; t0 += Chunk * nthr) {
+        V v[Chunk];
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
+        for (int j = 0; j < Chunk; ++j) {
             const int t = t0 + j * nthr;
             if (t < n) v[j] = get(t);
         }
 #pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
+        for (int j = 0; j < Chunk; ++j) {
             const int t = t0 + j * nthr;
             if (t < n) put(t, v[j]);
         }
@@ -276,10 +332,11 @@ GPVI_SPEC_FN void chunked(int n, int tid, int nthr, Get get, Put put)
 template <class Load>
 GPVI_SPEC_FN void rows_load(Cx* X, int np, int ntx, int ntz, int pair0, Load p1, int tid, int nthr)
 {
+    const Div by = divider(ntx);
     chunked(
         np * ntx, tid, nthr,
         [&](int t) {
-            const int q = t / ntx, ix = t - q * ntx;
+            const int q = quot(t, by), ix = t - q * ntx;
             const int iz = 2 * (pair0 + q);
             const double a = iz < ntz ? p1(iz, ix) : 0.0;
             const double b = iz + 1 < ntz ? p1(iz + 1, ix) : 0.0;
@@ -293,8 +350,9 @@ GPVI_SPEC_FN void rows_load(Cx* X, int np, int ntx, int ntz, int pair0, Load p1,
 template <class Store>
 GPVI_SPEC_FN void rows_unpack(const Cx* Z, int np, int ntx, int ntz, int nc, int pair0, Store st, int tid, int nthr)
 {
+    const Div by = divider(nc);
     for (int t = tid; t < np * nc; t += nthr) {
-        const int q = t / nc, f = t - q * nc;
+        const int q = quot(t, by), f = t - q * nc;
         const int iz = 2 * (pair0 + q);
         if (iz >= ntz) continue;
         const Cx zf = Z[q * ntx + f];
@@ -309,15 +367,16 @@ GPVI_SPEC_FN void rows_unpack(const Cx* Z, int np, int ntx, int ntz, int nc, int
 template <class Load>
 GPVI_SPEC_FN void cols_load(Cx* X, int nc_tile, int ntz, int nc, int f0, Load sp, int tid, int nthr)
 {
+    const Div by = divider(nc_tile);
     chunked(
         nc_tile * ntz, tid, nthr,
         [&](int t) {
-            const int iz = t / nc_tile, c = t - iz * nc_tile;
+            const int iz = quot(t, by), c = t - iz * nc_tile;
             const int f = f0 + c;
             return f < nc ? sp(iz, f) : cx(0.0, 0.0);
         },
         [&](int t, Cx v) {
-            const int iz = t / nc_tile, c = t - iz * nc_tile;
+            const int iz = quot(t, by), c = t - iz * nc_tile;
             X[c * ntz + iz] = v;
         });
 }
@@ -326,8 +385,9 @@ GPVI_SPEC_FN void cols_load(Cx* X, int nc_tile, int ntz, int nc, int f0, Load sp
 template <class K>
 GPVI_SPEC_FN void cols_scale(Cx* X, int nc_tile, int ntz, int nc, int f0, K k, int tid, int nthr)
 {
+    const Div by = divider(ntz);
     for (int t = tid; t < nc_tile * ntz; t += nthr) {
-        const int c = t / ntz, iz = t - c * ntz;
+        const int c = quot(t, by), iz = t - c * ntz;
         const int f = f0 + c;
         if (f >= nc) continue;
         const double m = (double)(-k(iz, f));
@@ -339,8 +399,9 @@ GPVI_SPEC_FN void cols_scale(Cx* X, int nc_tile, int ntz, int nc, int f0, K k, i
 template <class Store>
 GPVI_SPEC_FN void cols_store(const Cx* X, int nc_tile, int ntz, int nc, int f0, Store st, int tid, int nthr)
 {
+    const Div by = divider(nc_tile);
     for (int t = tid; t < nc_tile * ntz; t += nthr) {
-        const int iz = t / nc_tile, c = t - iz * nc_tile;
+        const int iz = quot(t, by), c = t - iz * nc_tile;
         const int f = f0 + c;
         if (f < nc) st(iz, f, X[c * ntz + iz]);
     }
@@ -348,30 +409,34 @@ GPVI_SPEC_FN void cols_store(const Cx* X, int nc_tile, int ntz, int nc, int f0, 
 
 // Rows backward, load: sequence q of X = A + i B over the full length ntx,
 // where A, B are the Hermitian extensions of the half-spectrum rows
-// 2 (pair0 + q) and 2 (pair0 + q) + 1 (0 past ntz).
+// 2 (pair0 + q) and 2 (pair0 + q) + 1 (0 past ntz).  Each half-spectrum value
+// is read once, for the elements f and ntx - f.
 template <class Load>
 GPVI_SPEC_FN void rows_repack(Cx* X, int np, int ntx, int ntz, int pair0, Load sp, int tid, int nthr)
 {
-    chunked(
-        np * ntx, tid, nthr,
+    struct Two {
+        Cx a, b;
+    };
+    const int nc = ntx / 2 + 1;
+    const Div by = divider(nc);
+    chunked<2>(
+        np * nc, tid, nthr,
         [&](int t) {
-            const int q = t / ntx, f = t - q * ntx;
+            const int q = quot(t, by), f = t - q * nc;
             const int iz = 2 * (pair0 + q);
-            const bool hi = 2 * f > ntx;
-            const int g = hi ? ntx - f : f;
-            Cx a = iz < ntz ? sp(iz, g) : cx(0.0, 0.0);
-            Cx b = iz + 1 < ntz ? sp(iz + 1, g) : cx(0.0, 0.0);
-            if (g == 0 || 2 * g == ntx) {
-                a.im = 0.0;
-                b.im = 0.0;
-            }
-            if (hi) {
-                a.im = -a.im;
-                b.im = -b.im;
-            }
-            return cx(a.re - b.im, a.im + b.re);
+            Two v;
+            v.a = iz < ntz ? sp(iz, f) : cx(0.0, 0.0);
+            v.b = iz + 1 < ntz ? sp(iz + 1, f) : cx(0.0, 0.0);
+            return v;
         },
-        [&](int t, Cx v) { X[t] = v; });
+        [&](int t, Two v) {
+            const int q = quot(t, by), f = t - q * nc;
+            const bool self = f == 0 || 2 * f == ntx;   // its own mirror image
+            if (self) v.a.im = v.b.im = 0.0;
+            Cx* x = X + q * ntx;
+            x[f] = cx(v.a.re - v.b.im, v.a.im + v.b.re);
+            if (!self) x[ntx - f] = cx(v.a.re + v.b.im, v.b.re - v.a.im);
+        });
 }
 
 }  // namespace spec
