@@ -349,7 +349,12 @@ constexpr int kResChunk = 256;       // time steps per launch
 struct ResChoice {
     bool ok;
     ResPlan plan;
+    double res_us;   // modelled time of a resident step
 };
+double step_launch_us(int lc, double points)
+{
+    return kStepUs + kStepUsPerMpoint * (1 + kStepUsPerLc * (lc - 4)) * 1e-6 * points;
+}
 std::mutex g_res_mu;
 std::map<std::tuple<int, int, int, int, int>, ResChoice> g_res_plans;
 constexpr size_t kMaxResPlans = 256;
@@ -390,9 +395,8 @@ void res_choose(const Geom& g, int units, ResChoice* out)
     if (out->ok) {
         const int n = out->plan.slabs;
         const double halo = n > 1 ? kResHaloRows * 2 * out->plan.hr * g.ntx / 256.0 : 0.0;
-        const double res_us = rounds(n) * (kResRoundUs + kResRowUs * halo) + kResRowUs * best;
-        const double step_us = kStepUs + kStepUsPerMpoint * (1 + kStepUsPerLc * (g.lc - 4)) * 1e-6 * units * g.ntx * g.ntz;
-        out->ok = res_us < step_us;
+        out->res_us = rounds(n) * (kResRoundUs + kResRowUs * halo) + kResRowUs * best;
+        out->ok = out->res_us < step_launch_us(g.lc, (double)units * g.ntx * g.ntz);
     }
     if (g_res_plans.size() >= kMaxResPlans) g_res_plans.clear();
     g_res_plans[key] = *out;
@@ -422,7 +426,8 @@ struct BatchLayout {
 
 // model_only: forward modelling without a wavefield store (records only);
 // no adjoint fields, checkpoints, store or private gradients are laid out.
-void batch_layout(const Geom& g, const Sched& sc, int nsample, bool tables, char* base, BatchLayout* L,
+// halo: lay out what resident steps need, where the batch takes them.
+void batch_layout(const Geom& g, const Sched& sc, int nsample, bool tables, bool halo, char* base, BatchLayout* L,
                   bool model_only = false)
 {
     Bump b{base};
@@ -436,7 +441,7 @@ void batch_layout(const Geom& g, const Sched& sc, int nsample, bool tables, char
     auto org = [&](float* p) { return p ? p + g.origin : nullptr; };
     ResChoice rc;
     rc.ok = false;
-    if (tables) res_choose(g, (int)U, &rc);
+    if (halo) res_choose(g, (int)U, &rc);
     L->vel_stride = rc.ok ? 2 * g.fe : g.fe;
     L->vel = org(b.take<float>((size_t)(nsample * L->vel_stride)));
     L->halo = nullptr;
@@ -973,7 +978,7 @@ size_t gpvi_fwi2d_batch_workspace_bytes(const gpvi_fwi2d_params* p, int nsample,
     make_geom(p, kDefaultVariant, tuning().tb, &g);   // the layout is the same for every variant
     Sched sc = make_sched(g, ckpt_interval);
     BatchLayout L;
-    batch_layout(g, sc, nsample, true, nullptr, &L);
+    batch_layout(g, sc, nsample, true, true, nullptr, &L);
     return L.bytes;
 }
 
@@ -984,7 +989,7 @@ size_t gpvi_fwi2d_model_workspace_bytes(const gpvi_fwi2d_params* p, int nsample)
     make_geom(p, kDefaultVariant, tuning().tb, &g);
     Sched sc = make_sched(g, 0);
     BatchLayout L;
-    batch_layout(g, sc, nsample, true, nullptr, &L, true);
+    batch_layout(g, sc, nsample, true, true, nullptr, &L, true);
     return L.bytes;
 }
 
@@ -1096,33 +1101,51 @@ int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, in
     return 0;
 }
 
-// The batch's steps with the fields on the chip: launches of up to kResChunk
-// steps, each within one pass (forward, a segment's recompute, an adjoint
-// stretch).
-int res_run(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom& g, const Sched& sc, const JobDesc& j,
-            const BatchLayout& L, const ResPlan& plan, int capacity)
-{
-    const int64_t units = (int64_t)nsample * g.ns;
-    unsigned* const tickets = reinterpret_cast<unsigned*>(L.halo + units * L.halo_stride);
-    HIP_TRY(launch_zero(st, reinterpret_cast<float*>(L.halo), 2 * units * L.halo_stride + kResTickets));
-    HIP_TRY(launch_vdt2(st, L.vel, L.vel + g.fe, p->dt, (int64_t)g.ntz * g.pitch, L.vel_stride, nsample));
-    UnitDesc sd;
-    std::memset(&sd, 0, sizeof sd);
-    sd.nt = g.nt; sd.tb = 1; sd.nseg = sc.nseg; sd.ckpt = sc.ckpt; sd.last_len = sc.last_len;
-    auto at = [&](int s) { return decode_step(sd, s + j.s_off); };
+// The resident steps of a batch or an engine job.
+struct ResRun {
     ResArgs a;
-    a.units = L.units;
+    UnitDesc sd;          // what decode_step reads
+    unsigned* tickets;
+    int used;             // launches since the tickets were cleared
+    int lc, s_off, total;
+};
+
+// Clears the exchange words and makes (v dt)^2, in stream order.
+int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom& g, const Sched& sc, const JobDesc& j,
+              const BatchLayout& L, const UnitDesc* units, const ResPlan& plan, int capacity, ResRun* run)
+{
+    const int64_t n = (int64_t)nsample * g.ns;
+    HIP_TRY(launch_zero(st, reinterpret_cast<float*>(L.halo), 2 * n * L.halo_stride + kResTickets));
+    HIP_TRY(launch_vdt2(st, L.vel, L.vel + g.fe, p->dt, (int64_t)g.ntz * g.pitch, L.vel_stride, nsample));
+    std::memset(&run->sd, 0, sizeof run->sd);
+    run->sd.nt = g.nt; run->sd.tb = 1; run->sd.nseg = sc.nseg; run->sd.ckpt = sc.ckpt; run->sd.last_len = sc.last_len;
+    run->tickets = reinterpret_cast<unsigned*>(L.halo + n * L.halo_stride);
+    run->used = 0;
+    run->lc = g.lc;
+    run->s_off = j.s_off;
+    run->total = j.total;
+    ResArgs& a = run->a;
+    a.units = units;
     a.halo = L.halo;
     a.halo_stride = L.halo_stride;
     a.vdt2_off = (int)(g.fe * sizeof(float));
     a.plan = plan;
-    a.nunit = (int)units;
-    a.clusters = std::max(1, std::min((int)units, capacity / plan.slabs));
-    int used = 0;
-    for (int s = 0; s < j.total;) {
+    a.nunit = (int)n;
+    a.clusters = std::max(1, std::min((int)n, capacity / plan.slabs));
+    return 0;
+}
+
+// Steps [s, end) with the fields on the chip: launches of up to kResChunk
+// steps, each within one pass (forward, a segment's recompute, an adjoint
+// stretch).
+int res_steps(hipStream_t st, ResRun* run, int s, int end)
+{
+    auto at = [&](int i) { return decode_step(run->sd, i + run->s_off); };
+    end = std::min(end, run->total);
+    while (s < end) {
         const StepInfo first = at(s);
         int n = 1;
-        while (n < kResChunk && s + n < j.total) {
+        while (n < kResChunk && s + n < end) {
             const StepInfo q = at(s + n);
             if (q.mode != first.mode || q.seg != first.seg) {
                 // the forward pass runs through its checkpoint segments
@@ -1130,14 +1153,14 @@ int res_run(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom&
             }
             ++n;
         }
-        if (used == kResTickets) {
-            HIP_TRY(launch_zero(st, reinterpret_cast<float*>(tickets), kResTickets));
-            used = 0;
+        if (run->used == kResTickets) {
+            HIP_TRY(launch_zero(st, reinterpret_cast<float*>(run->tickets), kResTickets));
+            run->used = 0;
         }
-        a.ticket = tickets + used++;
-        a.s0 = s + j.s_off;
-        a.n = n;
-        HIP_TRY(launch_resident(st, g.lc, first.mode == kAdj, a));
+        run->a.ticket = run->tickets + run->used++;
+        run->a.s0 = s + run->s_off;
+        run->a.n = n;
+        HIP_TRY(launch_resident(st, run->lc, first.mode == kAdj, run->a));
         s += n;
     }
     return 0;
@@ -1237,9 +1260,9 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     const bool model_only = phase == GPVI_PHASE_FORWARD && (flags & GPVI_FLAG_NO_STORE);
     Sched sc = make_sched(g, model_only ? 0 : ckpt_interval);
     BatchLayout L;
-    batch_layout(g, sc, nsample, true, nullptr, &L, model_only);
+    batch_layout(g, sc, nsample, true, true, nullptr, &L, model_only);
     if ((rc = check_workspace(workspace, workspace_bytes, L.bytes))) return rc;
-    batch_layout(g, sc, nsample, true, (char*)workspace, &L, model_only);
+    batch_layout(g, sc, nsample, true, true, (char*)workspace, &L, model_only);
     hipStream_t st = (hipStream_t)stream;
     if (phase != GPVI_PHASE_ADJOINT) {
         if ((rc = job_setup(st, p, g, vel_inner, L.vel, L.vel_stride, L.wav, L.zero, nsample))) return rc;
@@ -1310,7 +1333,9 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
         return 0;
     }
     if (resident) {
-        if ((rc = res_run(st, p, nsample, g, sc, j, L, rcho.plan, res_cap))) return rc;
+        ResRun run;
+        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho.plan, res_cap, &run))) return rc;
+        if ((rc = res_steps(st, &run, 0, run.total))) return rc;
         if (phase != GPVI_PHASE_FORWARD)
             HIP_TRY(launch_grad_reduce(st, L.gpriv, L.grad_stride, grad, g.ns, g.ni, nsample));
         if (phase != GPVI_PHASE_ADJOINT && misfit)
@@ -1442,6 +1467,9 @@ struct EngineJob {
     const float* obs;
     hipEvent_t done;
     bool cancelled;
+    bool resident, res_now;   // can run resident steps; runs them in this advance
+    double res_us;            // modelled time of one
+    ResRun run;
 };
 
 }  // namespace
@@ -1450,6 +1478,7 @@ struct gpvi_engine {
     hipStream_t stream;
     int device;
     int max_units, max_tiles, grid, variant, seg_steps, tb;
+    bool resident;   // made with no launch shape set
     UnitDesc* units;
     TileRef* tiles;
     StepCtl* ctl;
@@ -1486,7 +1515,8 @@ void engine_free_slots(gpvi_engine* e, int first, int n)
 int engine_rebuild(gpvi_engine* e)
 {
     int n4[4] = {0, 0, 0, 0}, o4[4] = {0, 0, 0, 0};
-    for (const auto& jb : e->active) n4[jb.g.lc - 4] += jb.nunit * jb.g.tpu;
+    for (const auto& jb : e->active)
+        if (!jb.res_now) n4[jb.g.lc - 4] += jb.nunit * jb.g.tpu;
     int off = 0;
     for (int g = 0; g < 4; ++g) {
         o4[g] = off;
@@ -1494,13 +1524,47 @@ int engine_rebuild(gpvi_engine* e)
     }
     int cur[4] = {o4[0], o4[1], o4[2], o4[3]};
     for (auto& jb : e->active) {
-        jb.j.tile0 = cur[jb.g.lc - 4];
-        cur[jb.g.lc - 4] += jb.nunit * jb.g.tpu;
+        // (the tiles of jobs on resident steps lie behind those of the launches)
+        int& at = jb.res_now ? off : cur[jb.g.lc - 4];
+        jb.j.tile0 = at;
+        at += jb.nunit * jb.g.tpu;
         HIP_TRY(launch_build_units(e->stream, jb.j, e->units, e->tiles));
     }
     HIP_TRY(launch_ctl_set(e->stream, e->ctl, (int)e->gstep, n4, o4));
     e->dirty = false;
     return 0;
+}
+
+// Which jobs advance by resident steps: those that can, one after the other,
+// when that and the step launches of the rest are modelled faster than one
+// launch per step for all of them.  A few jobs: 48 units of 128x228 padded
+// points for 600 time steps and 24 of 228x428 for 300 took 33.0 ms by
+// launches and take 13.9 ms; a stream at half load 46 and 27 ms (median).
+// Many small jobs share a launch better: at saturation the choice stays with
+// the launches (317 samples/s, 315 without resident steps).
+void engine_pick(gpvi_engine* e)
+{
+    double all = 0, rest = 0, res = 0;   // step launches of all jobs, of the others; resident steps
+    int lc_all = 4, lc_rest = 4;
+    bool others = false;
+    for (const auto& jb : e->active) {
+        const double points = (double)jb.nunit * jb.g.ntx * jb.g.ntz;
+        all += points;
+        lc_all = std::max(lc_all, jb.g.lc);
+        if (jb.resident) {
+            res += jb.res_us;
+        } else {
+            rest += points;
+            lc_rest = std::max(lc_rest, jb.g.lc);
+            others = true;
+        }
+    }
+    const bool use = res + (others ? step_launch_us(lc_rest, rest) : 0) < step_launch_us(lc_all, all);
+    for (auto& jb : e->active) {
+        const bool now = use && jb.resident;
+        if (now != jb.res_now) e->dirty = true;
+        jb.res_now = now;
+    }
 }
 
 int engine_finalize(gpvi_engine* e, EngineJob& jb)
@@ -1531,6 +1595,7 @@ int gpvi_engine_create(void* stream, int max_units, int max_tiles, gpvi_engine**
     e->max_tiles = max_tiles;
     e->variant = t.variant >= 0 ? t.variant : kDefaultVariant;
     e->tb = t.tb;
+    e->resident = t.variant < 0 && t.grid == 0 && t.tb == 1;
     e->seg_steps = t.graph_steps;
     e->grid = t.grid > 0 ? std::max(8, t.grid / 8 * 8) : 0;
     e->gstep = 0;
@@ -1604,10 +1669,19 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
     EngineJob jb;
     make_geom(p, e->variant, e->tb, &jb.g);
     jb.sc = make_sched(jb.g, ckpt_interval);
-    batch_layout(jb.g, jb.sc, nsample, false, nullptr, &jb.L);
-    if ((rc = check_workspace(workspace, workspace_bytes, jb.L.bytes))) return rc;
-    batch_layout(jb.g, jb.sc, nsample, false, (char*)workspace, &jb.L);
     jb.nunit = nsample * jb.g.ns;
+    ResChoice rcho;
+    rcho.ok = false;
+    if (e->resident) res_choose(jb.g, jb.nunit, &rcho);
+    const int res_cap = rcho.ok ? std::min(res_capacity(jb.g.lc), stream_cus(e->stream)) : 0;
+    batch_layout(jb.g, jb.sc, nsample, false, true, nullptr, &jb.L);
+    // (a workspace without the room for the exchange words keeps the launches)
+    jb.resident = rcho.ok && res_cap >= rcho.plan.slabs && jb.L.bytes <= workspace_bytes;
+    batch_layout(jb.g, jb.sc, nsample, false, jb.resident, nullptr, &jb.L);
+    if ((rc = check_workspace(workspace, workspace_bytes, jb.L.bytes))) return rc;
+    batch_layout(jb.g, jb.sc, nsample, false, jb.resident, (char*)workspace, &jb.L);
+    jb.res_now = false;
+    jb.res_us = rcho.ok ? rcho.res_us : 0;
     int tiles_now = 0;
     for (const auto& a : e->active) tiles_now += a.nunit * a.g.tpu;
     if (tiles_now + jb.nunit * jb.g.tpu > e->max_tiles)
@@ -1630,6 +1704,12 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
         (void)hipEventDestroy(jb.done);
         return fail(GPVI_ERR_CAPACITY, "step counter at %lld: let the engine drain before submitting", e->gstep);
     }
+    if (jb.resident && (rc = res_begin(e->stream, p, nsample, jb.g, jb.sc, jb.j, jb.L, e->units + first, rcho.plan,
+                                       res_cap, &jb.run))) {
+        engine_free_slots(e, first, jb.nunit);
+        (void)hipEventDestroy(jb.done);
+        return rc;
+    }
     jb.j.unit0 = first;
     jb.j.start = (int)e->gstep;
     jb.end_step = e->gstep + jb.j.total;
@@ -1650,10 +1730,12 @@ int gpvi_engine_advance(gpvi_engine* e, int nsteps)
     if (!e) return fail(GPVI_ERR_INVALID, "NULL engine");
     TraceRange tr("gpvi_engine_advance %zu jobs", e->active.size());
     int rc;
+    if (nsteps > 0) engine_pick(e);
     if (e->dirty && (rc = engine_rebuild(e))) return rc;
     if (e->active.empty() || nsteps <= 0) return 0;
     int mask = 0;
-    for (const auto& jb : e->active) mask |= 1 << (jb.g.lc - 4);
+    for (const auto& jb : e->active)
+        if (!jb.res_now) mask |= 1 << (jb.g.lc - 4);
     // Items 0: every launch uses the resident grid, so the graph survives
     // changes of the job set.
     GraphKey key{e->units, e->tiles, e->ctl, e->grid, e->tb, mask, e->seg_steps, e->device, {0, 0, 0, 0}};
@@ -1661,19 +1743,27 @@ int gpvi_engine_advance(gpvi_engine* e, int nsteps)
     for (const auto& jb : e->active) pending = std::max(pending, jb.end_step - e->gstep);
     const long long todo = std::min<long long>(nsteps, pending);
     const int reps = (int)((todo + e->seg_steps - 1) / e->seg_steps);
-    for (int r = 0; r < reps; ++r) {
+    // Without step launches, the segments of one resident launch together.
+    const int most = mask ? 1 : std::max(1, kResChunk / e->seg_steps);
+    for (int r = 0; r < reps;) {
+        const int segs = std::min(most, reps - r);
         // Keep at most three segments queued ahead of the device.
         while (e->inflight.size() >= 3) {
             HIP_TRY(hipEventSynchronize(e->inflight.front()));
             (void)hipEventDestroy(e->inflight.front());
             e->inflight.erase(e->inflight.begin());
         }
-        if ((rc = run_graph(key, e->stream, 1))) return rc;
+        if (mask && (rc = run_graph(key, e->stream, 1))) return rc;
+        const long long to = e->gstep + (long long)segs * e->seg_steps;
+        for (auto& jb : e->active)
+            if (jb.res_now && (rc = res_steps(e->stream, &jb.run, (int)(e->gstep - jb.j.start), (int)(to - jb.j.start))))
+                return rc;
         hipEvent_t ev;
         HIP_TRY(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
         HIP_TRY(hipEventRecord(ev, e->stream));
         e->inflight.push_back(ev);
-        e->gstep += e->seg_steps;
+        e->gstep = to;
+        r += segs;
     }
     int ncomplete = 0;
     for (size_t i = 0; i < e->active.size();) {

@@ -2,7 +2,9 @@
 
 The engine advances every active job by one time step per launch: all
 (sample, shot) units of all jobs, of any grid size, share each launch
-(replayed as graph segments).  Jobs join at a step boundary and leave when
+(replayed as graph segments).  A few jobs advance by resident steps instead
+(fields on the chip, one launch per job for many steps), and a job may change
+from one to the other between two advances.  Jobs join at a step boundary and leave when
 their last step is done; their finalising kernels (shot-ordered gradient
 sum, misfit) are queued right behind.  Inputs, outputs and the per-job
 workspace are caller-owned device memory (torch tensors here).
