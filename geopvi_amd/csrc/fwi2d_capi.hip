@@ -588,10 +588,14 @@ int stream_cus(hipStream_t st)
 // items until the list is done.
 // Tile variant of a batched call when none is set: the longest strip
 // segments (24, 16, then 8 rows) that still give each lane's launch at least
-// one resident grid of work items.  Shorter segments mean more, smaller items,
-// so a small batch fills the GPU; on full batches the 24-row segments are the
-// fastest.  c1, two lanes: one sample 10.5 -> 16.3 samples/s with 8 rows,
-// two 18.6 -> 23.1, four 28.4 -> 29.5; eight and more keep 24 rows.
+// three quarters of a resident grid of work items.  Shorter segments mean
+// more, smaller items, so a small batch fills the GPU; on full batches the
+// 24-row segments are the fastest.  Two lanes, us per step, items per lane in
+// resident grids in brackets: 24 units of 328x928 padded points 16 rows (0.66)
+// 30.2, 8 rows 29.1; 30 units 16 rows (0.82) 33.8, 8 rows 38.7; 60 units of
+// 178x628 16 rows (0.64) 33.5, 8 rows 31.4; 32 units of 334x634, Lc 6, 16 rows
+// (0.98) 31.1, 8 rows 33.4; 80 units of 228x728 24 rows (0.85) 51.1, 16 rows
+// 52.6.
 int auto_variant(const gpvi_fwi2d_params* p, int nsample, const Tuning& tn)
 {
     const int units = nsample * p->ns;
@@ -602,7 +606,7 @@ int auto_variant(const gpvi_fwi2d_params* p, int nsample, const Tuning& tn)
         Geom g;
         make_geom(p, v, tn.tb, &g);
         if (g.lc == 0) return kDefaultVariant;   // pseudo-spectral: no strip items
-        if ((int64_t)per_lane * g.tpu >= 4 * (int64_t)step_capacity(g.lc, g.tb)) return v;
+        if ((int64_t)per_lane * g.tpu >= 3 * (int64_t)step_capacity(g.lc, g.tb)) return v;   // (4 items a workgroup)
     }
     return 3;
 }
