@@ -23,6 +23,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 
 namespace gpvi {
 
@@ -134,7 +135,8 @@ GPVI_RES_FN void res_item_rows(const ResSlab& s, const ResItem& it, int* start, 
 
 // ---------------------------------------------------------------------------
 // Host side: building a plan.  Costs are in units of one 64-point interior
-// row of one wavefront.
+// row of one wavefront; the values are the best over 18 batches of a random
+// search (within 8 % of the best plan of each).
 
 struct ResGeom {
     int ntx, ntz, lc, pml;
@@ -143,12 +145,13 @@ struct ResGeom {
 namespace res_detail {
 
 constexpr double kRow = 1.0, kRowZ = 2.55, kRowEdge = 0.3, kSide = 3.19, kSideZ = 3.3, kItem = 2.0;
-constexpr double kWave = 2.38, kHold = 0.0, kFixed = 4.0, kHalo = 0.9;
+constexpr double kWave = 2.38, kHold = 3.0, kFixed = 4.0, kHalo = 0.9;
 
 struct Work {
     ResItem it;
     double cost;
 };
+constexpr int kMaxWork = kResWaves * kResItems;   // items of a slab
 
 // Deal the items to the waves (wave w runs on SIMD w % 4): longest first, to
 // the least loaded SIMD and its least loaded wave, at most one held item per
@@ -156,8 +159,7 @@ struct Work {
 // slots), < 0: it does not fit.
 inline double deal(const Work* w, int n, ResItem (*out)[kResItems])
 {
-    int order[256];
-    if (n > 256) return -1;
+    int order[kMaxWork];
     for (int i = 0; i < n; ++i) order[i] = i;
     std::stable_sort(order, order + n, [&](int a, int b) {
         return w[a].it.hold != w[b].it.hold ? w[a].it.hold > w[b].it.hold : w[a].cost > w[b].cost;
@@ -188,10 +190,6 @@ inline double deal(const Work* w, int n, ResItem (*out)[kResItems])
     return m;
 }
 
-struct Pieces {
-    int strip, side, z, zside;
-};
-
 // Cost of `r` rows of a strip's z zone, the first one d rows from the edge.
 inline double zone_cost(const ResGeom& g, int d, int r)
 {
@@ -207,53 +205,75 @@ inline double zone_cost(const ResGeom& g, int d, int r)
     return c + kRow * ((left + rb - 1) / rb * rb);
 }
 
-// The items of a slab of n rows, the first one z0 rows from the edge: rows
-// [0, tb) are z rows, and so are the last be rows (a whole-grid slab).
-inline int slab_items(const ResGeom& g, const ResPlan& p, int z0, int n, int tb, int be, const Pieces& pc, Work* out,
-                      int* held)
+// A slab of n rows, the first one z0 rows from the edge: rows [0, tb) are z
+// rows, and so are the last be rows (a whole-grid slab).  Its z items, each
+// strip's z rows in `strip` pieces and each side's in `side`, marched inward.
+// Pieces after the first hold their first four rows back (all of a shorter
+// one), and those lie in the band.  A cut is the one nearest to an equal share
+// of the cost or, late, the last one not far past it.  < 0: no such pieces.
+// Short pieces matter where few units leave most wavefronts idle and the
+// longest item is the step: with at least four rows in every later piece a
+// call on 120x200 with 4 shots took 11.8 ms instead of 9.7, 15 units of 61x97
+// 4.41 instead of 4.04.
+inline int zone_items(const ResGeom& g, const ResPlan& p, int z0, int n, int tb, int be, int strip, int side_pieces,
+                      bool late, Work* out, bool* held)
 {
     int c = 0;
-    *held = 0;
+    *held = false;
     for (int col = 0; col < p.strips + 2; ++col) {
         const bool side = col >= p.strips;
         const int x0 = side ? col - p.strips : p.wl + 64 * col;
         const int wd = side ? (x0 ? p.wr : p.wl) : 64;
-        // z rows, marched inward.  Pieces after the first begin with four band
-        // rows (held).
         for (int edge = 0; edge < 2; ++edge) {
             const int rows = edge ? be : tb, d0 = edge ? 0 : z0;
-            if (!rows) continue;
-            const int want = side ? pc.zside : pc.z;
+            const int want = side ? side_pieces : strip;
             int done = 0;
             for (int i = 0; i < want && done < rows; ++i) {
                 int r = rows - done;
+                const int at = d0 + done;
                 if (i + 1 < want) {
-                    // where the next piece may begin: an even number of band rows on, four of them left
-                    const double share = zone_cost(g, d0 + done, rows - done) / (want - i);
+                    const double share = zone_cost(g, at, r) / (want - i);
                     int cut = -1;
-                    for (int e = 4; done + e + 4 <= rows; ++e) {
-                        const int d = d0 + done + e;
-                        if (d < g.lc || d + 4 > g.pml) continue;
-                        if (!side && (d - std::max(g.lc, d0 + done)) % kResZBlock) continue;
-                        if (cut < 0 || zone_cost(g, d0 + done, e) <= share + kRowZ) cut = e;
+                    double off = 0;
+                    for (int e = late ? 4 : 1; e < r; ++e) {
+                        const int d = at + e, rest = i + 2 == want ? r - e : 2;
+                        if (d < g.lc || d + std::min(4, rest) > g.pml || (i > 0 && at + std::min(4, e) > g.pml)) continue;
+                        if (!side && (d - std::max(g.lc, at)) % kResZBlock) continue;   // (whole band blocks)
+                        const double cost = zone_cost(g, at, e), o = std::abs(cost - share);
+                        if (cut < 0 || (late ? cost <= share + kRowZ : o < off)) {
+                            cut = e;
+                            off = o;
+                        }
                     }
                     if (cut > 0) r = cut;
                 }
-                Work w;
+                if (i > 0 && at + std::min(4, r) > g.pml) return -1;
+                if (c == kMaxWork) return -1;
+                Work& w = out[c++];
                 w.it = ResItem{(uint16_t)x0, (int8_t)(edge ? -1 : 1), (uint8_t)(side ? kResSideZ : kResStripZ),
                                (uint8_t)(i > 0), (uint16_t)(edge ? n - 1 - done : done), (uint16_t)r};
-                w.cost = kItem + (side ? kSideZ * ((r * wd + 63) / 64) : zone_cost(g, d0 + done, r));
-                if (i > 0) *held = 1;
-                if (c < 256) out[c] = w;
-                ++c;
+                w.cost = kItem + (side ? kSideZ * ((r * wd + 63) / 64) : zone_cost(g, at, r));
+                if (i > 0) *held = true;
                 done += r;
             }
         }
-        const int m = n - tb - be;
-        if (m <= 0) continue;
+    }
+    return c;
+}
+
+// The slab's other items behind the c already there.
+inline int plain_items(const ResGeom& g, const ResPlan& p, int n, int tb, int be, int strip, int side_pieces, Work* out,
+                       int c)
+{
+    const int m = n - tb - be;
+    if (m <= 0) return c;
+    for (int col = 0; col < p.strips + 2; ++col) {
+        const bool side = col >= p.strips;
+        const int x0 = side ? col - p.strips : p.wl + 64 * col;
+        const int wd = side ? (x0 ? p.wr : p.wl) : 64;
         const int unit = side ? 1 : res_row_block(g.lc);      // rows advanced at a time
         const int blocks = (m + unit - 1) / unit;
-        const int k = std::min(side ? pc.side : pc.strip, blocks);
+        const int k = std::min(side ? side_pieces : strip, blocks);
         int done = 0;
         for (int i = 0; i < k; ++i) {
             // the first pieces march down from the top, the last one up from
@@ -261,16 +281,27 @@ inline int slab_items(const ResGeom& g, const ResPlan& p, int z0, int n, int tb,
             const int b = (i + 1) * blocks / k - i * blocks / k;
             const int rows = i == k - 1 ? m - done : std::min(m - done, b * unit);
             const bool up = i == k - 1 && k > 1;
-            Work w;
+            if (c == kMaxWork) return -1;
+            Work& w = out[c++];
             w.it = ResItem{(uint16_t)x0, (int8_t)(up ? -1 : 1), (uint8_t)(side ? kResSide : kResStrip), 0,
                            (uint16_t)(up ? tb + done + rows - 1 : tb + done), (uint16_t)rows};
             w.cost = kItem + (side ? kSide * ((rows * wd + 63) / 64) : kRow * ((rows + unit - 1) / unit * unit));
-            if (c < 256) out[c] = w;
-            ++c;
             done += rows;
         }
     }
     return c;
+}
+
+// What the items' cost alone makes of a step: equal shares on four SIMDs, and
+// the longest item's wavefront.
+inline double least_cost(const Work* w, int n)
+{
+    double sum = 0, top = 0;
+    for (int i = 0; i < n; ++i) {
+        sum += w[i].cost;
+        top = std::max(top, w[i].cost);
+    }
+    return std::max(sum / 4, kWave * top);
 }
 
 // The cheapest dealing of a slab's items; < 0: none costs less than `limit`.
@@ -278,31 +309,28 @@ inline double best_table(const ResGeom& g, const ResPlan& p, int z0, int n, int 
                          ResItem (*out)[kResItems], int* held, double limit)
 {
     double best = -1;
-    Work w[256];
+    Work w[kMaxWork];
     ResItem tmp[kResWaves][kResItems];
-    Pieces pc;
-    const bool zone = tb + be > 0;
-    for (pc.z = 1; pc.z <= (zone ? 3 : 1); ++pc.z)
-        for (pc.zside = 1; pc.zside <= (zone ? 3 : 1); ++pc.zside)
-            for (pc.strip = 1; pc.strip <= 16; pc.strip = pc.strip < 4 ? pc.strip + 1 : pc.strip * 2)
-                for (pc.side = 1; pc.side <= 8; pc.side *= 2) {
-                    int h = 0;
-                    const int c = slab_items(g, p, z0, n, tb, be, pc, w, &h);
-                    if (c > kResWaves * kResItems || c > 256) continue;
-                    const double wait = h ? kHold : 0.0;
-                    double sum = 0, top = 0;
-                    for (int i = 0; i < c; ++i) {
-                        sum += w[i].cost;
-                        top = std::max(top, w[i].cost);
+    const int most = tb + be > 0 ? 5 : 1;
+    for (int zs = 1; zs <= most; ++zs)
+        for (int zd = 1; zd <= most; ++zd)
+            for (int late = 0; late < (zs > 1 || zd > 1 ? 2 : 1); ++late) {
+                bool h;
+                const int nz = zone_items(g, p, z0, n, tb, be, zs, zd, late != 0, w, &h);
+                const double wait = h ? kHold : 0.0;
+                if (nz < 0 || least_cost(w, nz) + wait >= limit) continue;
+                for (int strip = 1; strip <= 16; strip = strip < 4 ? strip + 1 : strip * 2)
+                    for (int side = 1; side <= 8; side *= 2) {
+                        const int c = plain_items(g, p, n, tb, be, strip, side, w, nz);
+                        if (c < 0 || least_cost(w, c) + wait >= limit) continue;
+                        const double d = deal(w, c, tmp), m = d + wait;
+                        if (d < 0 || m >= limit) continue;
+                        best = limit = m;
+                        *held = h ? 1 : 0;
+                        for (int v = 0; v < kResWaves; ++v)
+                            for (int i = 0; i < kResItems; ++i) out[v][i] = tmp[v][i];
                     }
-                    if (std::max(sum / 4, kWave * top) + wait >= limit) continue;   // (four SIMDs)
-                    const double d = deal(w, c, tmp), m = d + wait;
-                    if (d < 0 || m >= limit) continue;
-                    best = limit = m;
-                    *held = h;
-                    for (int v = 0; v < kResWaves; ++v)
-                        for (int i = 0; i < kResItems; ++i) out[v][i] = tmp[v][i];
-                }
+            }
     return best;
 }
 

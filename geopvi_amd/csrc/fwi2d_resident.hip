@@ -481,7 +481,7 @@ __device__ __forceinline__ bool res_strip(const ResUnit& k, const ResStep& s, Ld
         }
     }
     if (hold) {
-        held.valid = ok ? 15u : 0u;
+        held.valid = ok ? (1u << min(cnt, 4)) - 1u : 0u;
         held.q[0] = f0 + start * k.P + ix;
         held.q[1] = held.q[0] + dz * k.P;
         held.step = 2 * dz * k.P;
