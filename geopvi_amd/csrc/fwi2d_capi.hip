@@ -337,9 +337,9 @@ Sched make_sched(const Geom& g, int ckpt_req)
 // batches; the resident side 6 % high, so that a near tie keeps the launches).
 // The fields of a wide grid fill the LDS with a few rows per slab, whose halo
 // rows then cost more than their own.  Measured, resident and per-step launch,
-// us a step: 2 units of 52x68 padded points 5.0 and 13.1, 64 of 148x228 7.6 and
-// 16.6, 20 of 228x428 8.2 and 15.5, 320 of them 86 and 124; 30 of 228x728 20
-// and 29, 80 of them 54 and 51; 16 of 328x928 26 and 27, 30 of them 49 and 36.
+// us a step: 2 units of 52x68 padded points 4.7 and 12.7, 64 of 148x228 7.4 and
+// 16.2, 20 of 228x428 8.1 and 15.3, 320 of them 86 and 123; 30 of 228x728 20
+// and 29, 80 of them 54 and 51; 16 of 328x928 26 and 27, 30 of them 49 and 34.
 constexpr double kResRoundUs = 1.06, kResRowUs = 0.072, kResHaloRows = 2.2;
 constexpr double kStepUs = 12.0, kStepUsPerMpoint = 3.0, kStepUsPerLc = 0.09;
 constexpr int kResCus = 256;
@@ -1543,7 +1543,7 @@ int engine_rebuild(gpvi_engine* e)
 // when that and the step launches of the rest are modelled faster than one
 // launch per step for all of them.  A few jobs: 48 units of 128x228 padded
 // points for 600 time steps and 24 of 228x428 for 300 took 33.0 ms by
-// launches and take 13.9 ms; a stream at half load 46 and 27 ms (median).
+// launches and take 13.8 ms; a stream at half load 46 and 27 ms (median).
 // Many small jobs share a launch better: at saturation the choice stays with
 // the launches (317 samples/s, 315 without resident steps).
 void engine_pick(gpvi_engine* e)

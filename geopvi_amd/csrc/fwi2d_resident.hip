@@ -28,7 +28,7 @@
 // gradient and the halo only.  One 1024-thread workgroup per CU, as the two
 // fields of a slab fill most of its LDS.  Microseconds a step of forward +
 // adjoint runs, one launch per step -> resident: 2 units of 52x68 padded points
-// 13.1 -> 5.0, 64 of 148x228 16.6 -> 7.6, 20 of 228x428 15.5 -> 8.2, 320 of
+// 12.7 -> 4.7, 64 of 148x228 16.2 -> 7.4, 20 of 228x428 15.3 -> 8.1, 320 of
 // them 124 -> 86.
 //
 // Arithmetic is the one of fwi2d_step.h, operation by operation.
