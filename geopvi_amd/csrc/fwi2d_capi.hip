@@ -355,6 +355,18 @@ double step_launch_us(int lc, double points)
 {
     return kStepUs + kStepUsPerMpoint * (1 + kStepUsPerLc * (lc - 4)) * 1e-6 * points;
 }
+// Slabs of a unit, at most.  Launches on different hardware queues run at the
+// same time, each with at most one cluster of which only some slabs have a CU:
+// with q queues, q (slabs - 1) < 256 always leaves one for a missing slab.
+int res_max_slabs()
+{
+    static const int most = [] {
+        const char* e = std::getenv("GPU_MAX_HW_QUEUES");
+        const int q = std::max(8, e ? std::atoi(e) : 0);
+        return std::max(1, std::min(kResMaxSlabs, kResCus / q));
+    }();
+    return most;
+}
 std::mutex g_res_mu;
 std::map<std::tuple<int, int, int, int, int>, ResChoice> g_res_plans;
 constexpr size_t kMaxResPlans = 256;
@@ -385,6 +397,7 @@ void res_choose(const Geom& g, int units, ResChoice* out)
     double best = 1e300;
     for (int slabs : order) {
         if (bound(slabs) >= best) break;
+        if (slabs > res_max_slabs()) continue;
         ResPlan p;
         const double c = res_make_plan(rg, slabs, &p, best / rounds(slabs) - res_fixed(rg, slabs));
         if (c < 0) continue;
