@@ -223,9 +223,10 @@ __global__ void psm_twiddle_kernel(Cx* __restrict__ tw, int ntx, int ntz)
     tw[i] = spec::cx(cs, sn);
 }
 
+template <int NT>
 __device__ inline void psm_table(Cx* T, const Cx* __restrict__ tw, int n)
 {
-    for (int m = threadIdx.x; m < spec::table_len(n); m += spec::kThreads) T[m] = tw[m];
+    for (int m = threadIdx.x; m < spec::table_len(n); m += NT) T[m] = tw[m];
 }
 
 // The plan's passes over nseq sequences, x -> y -> x ... (a barrier after
@@ -237,14 +238,14 @@ typedef const __attribute__((address_space(4))) double* RootPtr;
 #else
 typedef const double* RootPtr;
 #endif
-template <int MaxR>
+template <int MaxR, int NT>
 __device__ inline Cx* psm_transform(Cx* x, Cx* y, int nseq, const spec::Plan& p, const Cx* T, const Cx* tw, int sgn)
 {
     const RootPtr roots = (RootPtr)(uint64_t)tw;
     for (int i = 0; i < p.npass; ++i) {
         spec::run_pass<MaxR>(
             p.pass[i], x, y, nseq, p.n, T,
-            [&](int m) { return spec::cx(roots[2 * m], roots[2 * m + 1]); }, sgn, threadIdx.x, spec::kThreads);
+            [&](int m) { return spec::cx(roots[2 * m], roots[2 * m + 1]); }, sgn, threadIdx.x, NT);
         __syncthreads();
         Cx* t = x;
         x = y;
@@ -255,8 +256,8 @@ __device__ inline Cx* psm_transform(Cx* x, Cx* y, int nseq, const spec::Plan& p,
 
 // Rows forward: block (g, unit) transforms row pairs [g np, (g + 1) np) of
 // p1 and writes the half spectra of their rows.
-template <int MaxR>
-__global__ void __launch_bounds__(spec::kThreads)
+template <int MaxR, int NT>
+__global__ void __launch_bounds__(NT)
 psm_rows_fwd_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ spec_all, int64_t ustride,
                     const Cx* __restrict__ tw, spec::Plan px, int ntz, int np)
 {
@@ -269,21 +270,21 @@ psm_rows_fwd_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ 
     Cx* T = reinterpret_cast<Cx*>(psm_lds);
     Cx* X = T + spec::table_len(ntx);
     Cx* Y = X + np * ntx;
-    psm_table(T, tw, ntx);
+    psm_table<NT>(T, tw, ntx);
     const float* p1 = f.p1;
     const int pitch = u.pitch;
     spec::rows_load(X, np, ntx, ntz, pair0, [&](int iz, int ix) { return (double)p1[iz * pitch + ix]; },
-                    threadIdx.x, spec::kThreads);
+                    threadIdx.x, NT);
     __syncthreads();
-    const Cx* Z = psm_transform<MaxR>(X, Y, np, px, T, tw, +1);
+    const Cx* Z = psm_transform<MaxR, NT>(X, Y, np, px, T, tw, +1);
     spec::rows_unpack(Z, np, ntx, ntz, nc, pair0, [&](int iz, int fq, Cx v) { sp[iz * nc + fq] = v; },
-                      threadIdx.x, spec::kThreads);
+                      threadIdx.x, NT);
 }
 
 // Columns: block (g, unit) transforms spectrum columns [g ncol, (g + 1) ncol),
 // scales them by -|k|^2 and transforms them back.
-template <int MaxR>
-__global__ void __launch_bounds__(spec::kThreads)
+template <int MaxR, int NT>
+__global__ void __launch_bounds__(NT)
 psm_cols_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ spec_all, int64_t ustride,
                 const float* __restrict__ k, const Cx* __restrict__ tw, spec::Plan pz, int ntx, int ncol)
 {
@@ -303,17 +304,17 @@ psm_cols_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ spec
     Cx* T = reinterpret_cast<Cx*>(psm_lds);
     Cx* X = T + spec::table_len(ntz);
     Cx* Y = X + ncol * ntz;
-    psm_table(T, tw + ntx, ntz);
+    psm_table<NT>(T, tw + ntx, ntz);
     spec::cols_load(X, ncol, ntz, nc, f0, [&](int iz, int fq) { return sp[iz * nc + fq]; }, threadIdx.x,
-                    spec::kThreads);
+                    NT);
     __syncthreads();
-    Cx* Z = psm_transform<MaxR>(X, Y, ncol, pz, T, tw + ntx, +1);
+    Cx* Z = psm_transform<MaxR, NT>(X, Y, ncol, pz, T, tw + ntx, +1);
     spec::cols_scale(Z, ncol, ntz, nc, f0, [&](int iz, int fq) { return k[iz * ntx + fq]; }, threadIdx.x,
-                     spec::kThreads);
+                     NT);
     __syncthreads();
-    const Cx* W = psm_transform<MaxR>(Z, Z == X ? Y : X, ncol, pz, T, tw + ntx, -1);
+    const Cx* W = psm_transform<MaxR, NT>(Z, Z == X ? Y : X, ncol, pz, T, tw + ntx, -1);
     spec::cols_store(W, ncol, ntz, nc, f0, [&](int iz, int fq, Cx v) { sp[iz * nc + fq] = v; },
-                     threadIdx.x, spec::kThreads);
+                     threadIdx.x, NT);
 }
 
 // Rows backward and the point update: block (g, unit) transforms row pairs
@@ -322,8 +323,8 @@ psm_cols_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ spec
 // the block then also does the next step's rows-forward work on the p2 rows
 // it has just made, from LDS, and writes their half spectra over the ones it
 // read (each block reads and writes only its own rows).
-template <int MaxR>
-__global__ void __launch_bounds__(spec::kThreads)
+template <int MaxR, int NT>
+__global__ void __launch_bounds__(NT)
 psm_rows_inv_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ spec_all, int64_t ustride,
                     const Cx* __restrict__ tw, spec::Plan px, int ntz, int np, int chain)
 {
@@ -335,11 +336,11 @@ psm_rows_inv_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ 
     Cx* T = reinterpret_cast<Cx*>(psm_lds);
     Cx* X = T + spec::table_len(ntx);
     Cx* Y = X + np * ntx;
-    psm_table(T, tw, ntx);
+    psm_table<NT>(T, tw, ntx);
     spec::rows_repack(X, np, ntx, ntz, pair0, [&](int iz, int fq) { return sp[iz * nc + fq]; },
-                      threadIdx.x, spec::kThreads);
+                      threadIdx.x, NT);
     __syncthreads();
-    const Cx* Z = psm_transform<MaxR>(X, Y, np, px, T, tw, -1);
+    const Cx* Z = psm_transform<MaxR, NT>(X, Y, np, px, T, tw, -1);
     Cx* const W = Z == X ? Y : X;   // the next step's rows (chain)
     const FieldPtrs f = step_fields(u, si);
     const int64_t margin = (int64_t)kPadRows * u.pitch;
@@ -352,7 +353,7 @@ psm_rows_inv_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ 
     // points in flight, 107 registers, 135 us; four, 151 registers, 149 us).
     const int total = 2 * np * ntx;
     const spec::Div by_pair = spec::divider(2 * ntx);
-    for (int t = threadIdx.x; t < total; t += spec::kThreads) {
+    for (int t = threadIdx.x; t < total; t += NT) {
         const int q = spec::quot(t, by_pair), r = t - q * 2 * ntx;
         const int w = r >= ntx ? 1 : 0, ix = r - w * ntx;
         const int iz = 2 * (pair0 + q) + w;
@@ -367,9 +368,9 @@ psm_rows_inv_kernel(const UnitDesc* __restrict__ units, int s, Cx* __restrict__ 
     }
     if (!chain) return;   // uniform over the launch
     __syncthreads();
-    const Cx* F = psm_transform<MaxR>(W, W == X ? Y : X, np, px, T, tw, +1);
+    const Cx* F = psm_transform<MaxR, NT>(W, W == X ? Y : X, np, px, T, tw, +1);
     spec::rows_unpack(F, np, ntx, ntz, nc, pair0, [&](int iz, int fq, Cx v) { sp[iz * nc + fq] = v; },
-                      threadIdx.x, spec::kThreads);
+                      threadIdx.x, NT);
 }
 
 hipError_t launch_psm_wavenumber(hipStream_t st, float* k, int ntx, int ntz, float dx, float dz)
@@ -433,7 +434,8 @@ hipError_t launch_psm_twiddles(hipStream_t st, double* tw, int ntx, int ntz)
     return hipGetLastError();
 }
 
-hipError_t launch_psm_spectral(hipStream_t st, const UnitDesc* units, int nunit, int s, double* buf,
+template <int NT>
+static hipError_t launch_psm_spectral_nt(hipStream_t st, const UnitDesc* units, int nunit, int s, double* buf,
                                const float* k, const double* twd, int ntx, int ntz, bool first, bool chain)
 {
     spec::Plan px, pz;
@@ -449,31 +451,49 @@ hipError_t launch_psm_spectral(hipStream_t st, const UnitDesc* units, int nunit,
     const size_t lds_cols = sizeof(Cx) * ((size_t)spec::table_len(ntz) + (size_t)ntz * 2 * ncol);
     // instantiations by largest radix: 7, 11 or 13
     const int mx = spec::max_radix(px), mz = spec::max_radix(pz);
-    const dim3 rows(row_groups, nunit), cols(col_groups, nunit), blk(spec::kThreads);
+    const dim3 rows(row_groups, nunit), cols(col_groups, nunit), blk(NT);
     const int ch = chain ? 1 : 0;
     if (first) {
         if (mx <= 7)
-            hipLaunchKernelGGL(psm_rows_fwd_kernel<7>, rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np);
+            hipLaunchKernelGGL((psm_rows_fwd_kernel<7, NT>), rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np);
         else if (mx == 11)
-            hipLaunchKernelGGL(psm_rows_fwd_kernel<11>, rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np);
+            hipLaunchKernelGGL((psm_rows_fwd_kernel<11, NT>), rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np);
         else
-            hipLaunchKernelGGL(psm_rows_fwd_kernel<13>, rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np);
+            hipLaunchKernelGGL((psm_rows_fwd_kernel<13, NT>), rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np);
     }
     if (mz <= 7)
-        hipLaunchKernelGGL(psm_cols_kernel<7>, cols, blk, lds_cols, st, units, s, sp, ustride, k, tw, pz, ntx, ncol);
+        hipLaunchKernelGGL((psm_cols_kernel<7, NT>), cols, blk, lds_cols, st, units, s, sp, ustride, k, tw, pz, ntx, ncol);
     else if (mz == 11)
-        hipLaunchKernelGGL(psm_cols_kernel<11>, cols, blk, lds_cols, st, units, s, sp, ustride, k, tw, pz, ntx, ncol);
+        hipLaunchKernelGGL((psm_cols_kernel<11, NT>), cols, blk, lds_cols, st, units, s, sp, ustride, k, tw, pz, ntx, ncol);
     else
-        hipLaunchKernelGGL(psm_cols_kernel<13>, cols, blk, lds_cols, st, units, s, sp, ustride, k, tw, pz, ntx, ncol);
+        hipLaunchKernelGGL((psm_cols_kernel<13, NT>), cols, blk, lds_cols, st, units, s, sp, ustride, k, tw, pz, ntx, ncol);
     if (mx <= 7)
-        hipLaunchKernelGGL(psm_rows_inv_kernel<7>, rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np, ch);
+        hipLaunchKernelGGL((psm_rows_inv_kernel<7, NT>), rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np, ch);
     else if (mx == 11)
-        hipLaunchKernelGGL(psm_rows_inv_kernel<11>, rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np,
+        hipLaunchKernelGGL((psm_rows_inv_kernel<11, NT>), rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np,
                            ch);
     else
-        hipLaunchKernelGGL(psm_rows_inv_kernel<13>, rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np,
+        hipLaunchKernelGGL((psm_rows_inv_kernel<13, NT>), rows, blk, lds_rows, st, units, s, sp, ustride, tw, px, ntz, np,
                            ch);
     return hipGetLastError();
+}
+
+// Threads of a transform workgroup: with less than one workgroup a CU (in each
+// of a batch's two lanes) the latency of a phase counts, and twice the threads
+// have half the work in it; beyond, the 256-thread workgroups overlap better.
+// 256 and 512 threads, workgroups a lane in brackets, ms a call: 12 units of
+// 130x270 (198) 8.1 and 7.5, 12 of 130x210 (198) 10.4 and 9.4, 8 of 220x420
+// (220) 12.8 and 11.7; 13 of 169x351 (280) 29.0 and 29.9, 24 of 130x270 (396)
+// 12.5 and 13.7, 18 of 220x420 (495) 15.7 and 17.5.
+hipError_t launch_psm_spectral(hipStream_t st, const UnitDesc* units, int nunit, int s, double* buf,
+                               const float* k, const double* twd, int ntx, int ntz, bool first, bool chain)
+{
+    spec::Plan px, pz;
+    int np, ncol;
+    if (!psm_spectral_plans(ntx, ntz, &px, &pz, &np, &ncol)) return hipErrorInvalidValue;
+    const int64_t groups = (int64_t)(((ntz + 1) / 2 + np - 1) / np) * nunit;
+    return groups < 256 ? launch_psm_spectral_nt<2 * spec::kThreads>(st, units, nunit, s, buf, k, twd, ntx, ntz, first, chain)
+                            : launch_psm_spectral_nt<spec::kThreads>(st, units, nunit, s, buf, k, twd, ntx, ntz, first, chain);
 }
 
 }  // namespace gpvi
