@@ -382,33 +382,13 @@ void res_choose(const Geom& g, int units, ResChoice* out)
         *out = it->second;
         return;
     }
-    // Slab counts in the order of a lower bound on their time (equal work on
-    // every SIMD); the search ends where the bound passes the best plan found.
     const ResGeom rg{g.ntx, g.ntz, g.lc, g.pml};
-    const double work = res_work(rg) / 4;
-    auto rounds = [&](int slabs) {
-        const int at_once = std::max(1, kResCus / slabs);
-        return (double)((units + at_once - 1) / at_once);
-    };
-    auto bound = [&](int slabs) { return rounds(slabs) * (res_fixed(rg, slabs) + work / slabs); };
-    int order[kResMaxSlabs];
-    for (int i = 0; i < kResMaxSlabs; ++i) order[i] = i + 1;
-    std::stable_sort(order, order + kResMaxSlabs, [&](int a, int b) { return bound(a) < bound(b); });
-    double best = 1e300;
-    for (int slabs : order) {
-        if (bound(slabs) >= best) break;
-        if (slabs > res_max_slabs()) continue;
-        ResPlan p;
-        const double c = res_make_plan(rg, slabs, &p, best / rounds(slabs) - res_fixed(rg, slabs));
-        if (c < 0) continue;
-        best = rounds(slabs) * (res_fixed(rg, slabs) + c);
-        out->ok = true;
-        out->plan = p;
-    }
+    const double best = res_select_plan(rg, units, kResCus, res_max_slabs(), &out->plan);
+    out->ok = best >= 0;
     if (out->ok) {
         const int n = out->plan.slabs;
         const double halo = n > 1 ? kResHaloRows * 2 * out->plan.hr * g.ntx / 256.0 : 0.0;
-        out->res_us = rounds(n) * (kResRoundUs + kResRowUs * halo) + kResRowUs * best;
+        out->res_us = res_rounds(units, n, kResCus) * (kResRoundUs + kResRowUs * halo) + kResRowUs * best;
         out->ok = out->res_us < step_launch_us(g.lc, (double)units * g.ntx * g.ntz);
     }
     if (g_res_plans.size() >= kMaxResPlans) g_res_plans.clear();

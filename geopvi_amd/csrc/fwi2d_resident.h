@@ -126,11 +126,40 @@ GPVI_RES_FN void res_item_rows(const ResSlab& s, const ResItem& it, int* start, 
             c -= 1;
         }
     }
+    if (c <= 0) {   // the row was the item's only one (its start may lie outside the slab)
+        *start = 0; *step = 1; *count = 0;
+        return;
+    }
     if (s.flip) {
         a = s.n - 1 - a;
         d = -d;
     }
     *start = a; *step = d; *count = c;
+}
+
+// An item as the two words that a wavefront reads in every step, and back.
+GPVI_RES_FN void res_pack_item(const ResItem& it, int start, int step, int count, unsigned* w0, unsigned* w1)
+{
+    *w0 = (unsigned)it.x0 | (unsigned)it.kind << 16 | (step < 0 ? 1u << 18 : 0u) | (unsigned)it.hold << 19 |
+          (it.count ? 1u << 20 : 0u);
+    *w1 = ((unsigned)start & 0xffffu) | (unsigned)count << 16;
+}
+
+struct ResWords {
+    bool present, hold;
+    int x0, kind, step, start, count;
+};
+GPVI_RES_FN ResWords res_unpack_item(unsigned w0, unsigned w1)
+{
+    ResWords r;
+    r.present = w0 >> 20 & 1;
+    r.hold = w0 >> 19 & 1;
+    r.step = w0 >> 18 & 1 ? -1 : 1;
+    r.kind = (int)(w0 >> 16) & 3;
+    r.x0 = (int)(w0 & 0xffff);
+    r.start = (int)(w1 & 0xffff);
+    r.count = (int)(w1 >> 16);
+    return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -463,6 +492,38 @@ inline double res_make_plan(const ResGeom& g, int slabs, ResPlan* p, double limi
     }
     p->lds_bytes = res_lds_bytes(g.ntx, tallest, p->hr);
     return p->lds_bytes <= kResLdsBytes ? cost : -1;
+}
+
+// Rounds a launch takes over `units` units in `slabs` slabs each on `cus` CUs.
+inline double res_rounds(int units, int slabs, int cus)
+{
+    const int at_once = std::max(1, cus / slabs);
+    return (double)((units + at_once - 1) / at_once);
+}
+
+// The plan of least time, with at most `most` slabs; its cost (fixed part
+// included, all rounds), or < 0: none fits.  Slab counts are tried in the
+// order of a lower bound on their time (equal work on every SIMD); the search
+// ends where the bound passes the best plan found.
+inline double res_select_plan(const ResGeom& g, int units, int cus, int most, ResPlan* plan)
+{
+    const double work = res_work(g) / 4;
+    auto bound = [&](int slabs) { return res_rounds(units, slabs, cus) * (res_fixed(g, slabs) + work / slabs); };
+    int order[kResMaxSlabs];
+    for (int i = 0; i < kResMaxSlabs; ++i) order[i] = i + 1;
+    std::stable_sort(order, order + kResMaxSlabs, [&](int a, int b) { return bound(a) < bound(b); });
+    double best = 1e300;
+    for (int slabs : order) {
+        if (bound(slabs) >= best) break;
+        if (slabs > most) continue;
+        ResPlan p;
+        const double rounds = res_rounds(units, slabs, cus);
+        const double c = res_make_plan(g, slabs, &p, best / rounds - res_fixed(g, slabs));
+        if (c < 0) continue;
+        best = rounds * (res_fixed(g, slabs) + c);
+        *plan = p;
+    }
+    return best < 1e300 ? best : -1;
 }
 
 }  // namespace gpvi

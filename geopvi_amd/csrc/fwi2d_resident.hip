@@ -781,17 +781,17 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
             }
         }
     }
-    // The wave's items, decoded, in LDS: x0 | kind << 16 | upward << 18 | hold << 19 |
-    // present << 20, start | count << 16.
+    // The wave's items, decoded, in LDS.
     typedef __attribute__((address_space(3))) unsigned LdsU;
     LdsU* const my_items = (LdsU*)lds + 16 + wave * 2 * kResItems;
     if (lane < kResItems) {
         const ResItem item = pl.item[sl.table][wave][lane];
         int start, dz, cnt;
         res_item_rows(sl, item, &start, &dz, &cnt);
-        my_items[2 * lane] = (unsigned)item.x0 | (unsigned)item.kind << 16 | (dz < 0 ? 1u << 18 : 0u) |
-                             (unsigned)item.hold << 19 | (item.count ? 1u << 20 : 0u);
-        my_items[2 * lane + 1] = (unsigned)start | (unsigned)max(cnt, 0) << 16;
+        unsigned w0, w1;
+        res_pack_item(item, start, dz, cnt, &w0, &w1);
+        my_items[2 * lane] = w0;
+        my_items[2 * lane + 1] = w1;
     }
     k.taper = lds + 16 + 2 * kResWaves * kResItems;
     if (wave == 0 && lane < 32 && lane < u.pml0) k.taper[lane] = G(u.wtab)[lane];
@@ -879,17 +879,15 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
         held.step = 0;
         unsigned n0 = __builtin_amdgcn_readfirstlane(my_items[0]), n1 = __builtin_amdgcn_readfirstlane(my_items[1]);
         for (int q = 1; n0 >> 20 & 1; ++q) {
-            const unsigned d0 = n0, d1 = n1;
-            const int cnt = (int)(d1 >> 16);
+            const ResWords d = res_unpack_item(n0, n1);
+            const int cnt = d.count, start = d.start, x0 = d.x0, kind = d.kind, dz = d.step;
+            const bool hold = d.hold;
             n0 = 0;
             if (q < kResItems) {
                 n0 = __builtin_amdgcn_readfirstlane(my_items[2 * q]);
                 n1 = __builtin_amdgcn_readfirstlane(my_items[2 * q + 1]);
             }
             if (cnt == 0) continue;   // (the one row of an item that a shorter slab lacks)
-            const int start = (int)(d1 & 0xffff), x0 = (int)(d0 & 0xffff), kind = (int)(d0 >> 16) & 3;
-            const int dz = d0 >> 18 & 1 ? -1 : 1;
-            const bool hold = d0 >> 19 & 1;
             // rows from the edge of the z zone's first row in this item
             const int ec = e0 + (pl.slabs == 1 ? (dz > 0 ? start : n - 1 - start) : (sl.flip ? n - 1 - start : start));
             const int pos = x0 ? pos_r : pos_l, w = x0 ? pl.wr : pl.wl;
