@@ -968,15 +968,21 @@ int gpvi_fwi2d_forward_device(const gpvi_fwi2d_params* p, const float* vel_inner
 // ---------------------------------------------------------------------------
 // Batched solver
 
-size_t gpvi_fwi2d_batch_workspace_bytes(const gpvi_fwi2d_params* p, int nsample, int ckpt_interval)
+// Workspace of a batched call, with or without the room for resident steps.
+static size_t batch_bytes(const gpvi_fwi2d_params* p, int nsample, int ckpt_interval, bool resident)
 {
     if (validate(p) || nsample < 1) return 0;
     Geom g;
     make_geom(p, kDefaultVariant, tuning().tb, &g);   // the layout is the same for every variant
     Sched sc = make_sched(g, ckpt_interval);
     BatchLayout L;
-    batch_layout(g, sc, nsample, true, true, nullptr, &L);
+    batch_layout(g, sc, nsample, true, resident, nullptr, &L);
     return L.bytes;
+}
+
+size_t gpvi_fwi2d_batch_workspace_bytes(const gpvi_fwi2d_params* p, int nsample, int ckpt_interval)
+{
+    return batch_bytes(p, nsample, ckpt_interval, true);
 }
 
 size_t gpvi_fwi2d_model_workspace_bytes(const gpvi_fwi2d_params* p, int nsample)
@@ -1061,7 +1067,8 @@ int psm_plans(int ntz, int ntx, int batch, hipStream_t st, PsmPlans* out)
 // between.  A later forward call on the same address replaces the stamp.
 struct LayoutStamp {
     gpvi_fwi2d_params p;
-    int nsample, ckpt, variant, tb, resident;
+    int nsample, ckpt, variant, tb;
+    bool room;   // laid out for resident steps
     unsigned long long seq;
 };
 std::mutex g_stamp_mu;
@@ -1069,7 +1076,7 @@ std::map<const void*, LayoutStamp> g_stamps;
 unsigned long long g_stamp_seq = 0;
 constexpr size_t kMaxStamps = 4096;
 
-void layout_stamp_put(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, const Tuning& tn, bool resident)
+void layout_stamp_put(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, const Tuning& tn, bool room)
 {
     std::lock_guard<std::mutex> lk(g_stamp_mu);
     if (g_stamps.size() >= kMaxStamps && !g_stamps.count(ws)) {
@@ -1078,10 +1085,10 @@ void layout_stamp_put(const void* ws, const gpvi_fwi2d_params* p, int nsample, i
             if (it->second.seq < oldest->second.seq) oldest = it;
         g_stamps.erase(oldest);
     }
-    g_stamps[ws] = LayoutStamp{*p, nsample, ckpt, tn.variant, tn.tb, resident ? 1 : 0, ++g_stamp_seq};
+    g_stamps[ws] = LayoutStamp{*p, nsample, ckpt, tn.variant, tn.tb, room, ++g_stamp_seq};
 }
 
-int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, Tuning* tn, bool* resident)
+int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, int ckpt, Tuning* tn, bool* room)
 {
     std::lock_guard<std::mutex> lk(g_stamp_mu);
     auto it = g_stamps.find(ws);
@@ -1094,7 +1101,7 @@ int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, in
                                       "phase that prepared this workspace");
     tn->variant = s.variant;
     tn->tb = s.tb;
-    *resident = s.resident != 0;
+    *room = s.room;
     return 0;
 }
 
@@ -1240,13 +1247,14 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
         (phase != GPVI_PHASE_FORWARD && !grad))
         return fail(GPVI_ERR_INVALID, "NULL buffer");
     Tuning tn = tuning();
-    // Resident steps unless a launch shape of the per-step kernels is set.
-    bool resident = tn.variant < 0 && tn.grid == 0 && tn.tb == 1;
+    // Resident steps unless a launch shape of the per-step kernels is set; room:
+    // the workspace is laid out for them.
+    bool room = tn.variant < 0 && tn.grid == 0 && tn.tb == 1;
     // The adjoint phase continues the forward phase's workspace: it must use
     // the layout that phase used (tile variant and steps per launch fix the
     // strip width, band items, row shift, pitch and field stride), whatever
     // the process-wide tuning says now.
-    rc = phase == GPVI_PHASE_ADJOINT ? layout_stamp_get(workspace, p, nsample, ckpt_interval, &tn, &resident)
+    rc = phase == GPVI_PHASE_ADJOINT ? layout_stamp_get(workspace, p, nsample, ckpt_interval, &tn, &room)
                                      : 0;
     if (rc) return rc;
     if (tn.variant < 0) tn.variant = auto_variant(p, nsample, tn);
@@ -1256,20 +1264,27 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
         return fail(GPVI_ERR_INVALID, "pseudo-spectral batches hold at most 65535 (sample, shot) units");
     const bool model_only = phase == GPVI_PHASE_FORWARD && (flags & GPVI_FLAG_NO_STORE);
     Sched sc = make_sched(g, model_only ? 0 : ckpt_interval);
-    BatchLayout L;
-    batch_layout(g, sc, nsample, true, true, nullptr, &L, model_only);
-    if ((rc = check_workspace(workspace, workspace_bytes, L.bytes))) return rc;
-    batch_layout(g, sc, nsample, true, true, (char*)workspace, &L, model_only);
     hipStream_t st = (hipStream_t)stream;
+    ResChoice rcho;
+    rcho.ok = false;
+    if (room) res_choose(g, nsample * g.ns, &rcho);
+    const int res_cap = rcho.ok ? std::min(res_capacity(g.lc), stream_cus(st)) : 0;
+    const bool resident_fits = res_cap > 0 && res_cap >= rcho.plan.slabs;
+    BatchLayout L;
+    if (phase != GPVI_PHASE_ADJOINT && (room = resident_fits)) {
+        // (a workspace without the room keeps the launches: it may be sized for them)
+        batch_layout(g, sc, nsample, true, true, nullptr, &L, model_only);
+        room = L.bytes <= workspace_bytes;
+    }
+    batch_layout(g, sc, nsample, true, room, nullptr, &L, model_only);
+    if ((rc = check_workspace(workspace, workspace_bytes, L.bytes))) return rc;
+    batch_layout(g, sc, nsample, true, room, (char*)workspace, &L, model_only);
+    const bool resident = room && resident_fits;
     if (phase != GPVI_PHASE_ADJOINT) {
         if ((rc = job_setup(st, p, g, vel_inner, L.vel, L.vel_stride, L.wav, L.zero, nsample))) return rc;
     }
-    ResChoice rcho;
-    res_choose(g, nsample * g.ns, &rcho);
-    const int res_cap = resident && rcho.ok && L.halo ? std::min(res_capacity(g.lc), stream_cus(st)) : 0;
-    resident = res_cap > 0 && res_cap >= rcho.plan.slabs;
     if (phase == GPVI_PHASE_FORWARD && !model_only)
-        layout_stamp_put(workspace, p, nsample, ckpt_interval, tn, resident);
+        layout_stamp_put(workspace, p, nsample, ckpt_interval, tn, room);
     const int store = (phase == GPVI_PHASE_FORWARD && (flags & GPVI_FLAG_NO_STORE)) ? 0 : 1;
     JobDesc j = make_job(p, g, sc, nsample, L, record_obs, record_syn, run_fwi, phase, store);
     // Lanes: the units split into groups with contiguous runs of the tile
@@ -1428,7 +1443,7 @@ int gpvi_fwi2d_batch_static(const gpvi_fwi2d_params* p, int nsample, const float
     if (p->laplace_slover == 1)  // the transform plans would allocate
         return fail(GPVI_ERR_UNSUPPORTED, "gpvi_fwi2d_batch_static runs finite-difference jobs only");
     if (nsample < 1) return fail(GPVI_ERR_INVALID, "nsample=%d", nsample);
-    const size_t need = gpvi_fwi2d_batch_workspace_bytes(p, nsample, ckpt_interval);
+    const size_t need = batch_bytes(p, nsample, ckpt_interval, false);   // (by step launches)
     if (need > kStaticScratchBytes)
         return fail(GPVI_ERR_WORKSPACE,
                     "gpvi_fwi2d_batch_static: this job needs %zu bytes of scratch, the fixed scratch holds %zu "

@@ -110,7 +110,9 @@ int gpvi_fwi2d_forward_device(const gpvi_fwi2d_params *p, const float *vel_inner
  * reference's store); otherwise (p0, p1) checkpoints are kept every
  * ckpt_interval steps (rounded up to a multiple of nt_interval) and each
  * segment is recomputed during the adjoint.  misfit may be NULL; grad may be
- * NULL in GPVI_PHASE_FORWARD. */
+ * NULL in GPVI_PHASE_FORWARD.  The workspace size below has room for steps
+ * with the fields on the chip; a workspace that lacks only that room is
+ * accepted and every step is a launch. */
 size_t gpvi_fwi2d_batch_workspace_bytes(const gpvi_fwi2d_params *p, int nsample, int ckpt_interval);
 /* Workspace of a forward-modelling-only call (GPVI_PHASE_FORWARD with
  * GPVI_FLAG_NO_STORE; the reference's forward_2D, fdtd2D_modelling.c:356-675,
@@ -128,8 +130,8 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params *p, int nsample, const float *vel_i
  * GPVI_STATIC_SCRATCH_BYTES per GPU (held from library load until the
  * process ends) instead of an argument: the caller passes inputs and outputs
  * only.  Nothing is allocated.  A job whose workspace
- * (gpvi_fwi2d_batch_workspace_bytes) exceeds the scratch is refused with
- * GPVI_ERR_WORKSPACE; pseudo-spectral jobs with GPVI_ERR_UNSUPPORTED.  Every
+ * (gpvi_fwi2d_batch_workspace_bytes, or as much of it as one launch per step
+ * takes) exceeds the scratch is refused with GPVI_ERR_WORKSPACE; pseudo-spectral jobs with GPVI_ERR_UNSUPPORTED.  Every
  * call on a GPU uses that GPU's one scratch array: calls that overlap on one
  * GPU (two streams or two threads) race and must be serialised by the
  * caller. */
