@@ -38,6 +38,7 @@ SIGNATURES = {
     "gpvi_fwi2d_model_workspace_bytes": (_sz, [_P, _i]),
     "gpvi_fwi2d_batch": (_i, [_P, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _vp]),
     "gpvi_fwi2d_batch_static": (_i, [_P, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
+    "gpvi_fwi2d_resident_plan": (_i, [_P, _i, _vp] + [ctypes.POINTER(_i)] * 3),
     "gpvi_fwi2d_set_tuning": (_i, [_i, _i, _i]),
     "gpvi_fwi2d_get_tuning": (_i, [ctypes.POINTER(_i)] * 3),
     "gpvi_fwi2d_tile_shape": (_i, [_i, ctypes.POINTER(_i), ctypes.POINTER(_i)]),
@@ -55,6 +56,7 @@ SIGNATURES = {
     "gpvi_engine_cancel": (_i, [_vp, ctypes.c_longlong]),
     "gpvi_engine_active_jobs": (_i, [_vp]),
     "gpvi_engine_active_units": (_i, [_vp]),
+    "gpvi_engine_resident_jobs": (_i, [_vp]),
     "gpvi_engine_pending_steps": (_i, [_vp]),
     "gpvi_engine_sync": (_i, [_vp]),
     "fwi_2D": (None, [ctypes.c_char_p, ctypes.POINTER(ctypes.c_float), ctypes.POINTER(ctypes.c_float),

@@ -573,6 +573,17 @@ int stream_cus(hipStream_t st)
     return n ? n : 1 << 30;
 }
 
+// CUs that resident steps may use on `st` (0: they do not run there).
+int res_cus(const Geom& g, const ResChoice& c, hipStream_t st)
+{
+    if (!c.ok) return 0;
+    const int cus = std::min(res_capacity(g.lc), stream_cus(st));
+    return cus >= c.plan.slabs ? cus : 0;
+}
+
+// Groups of workgroups of a launch, one group per unit at a time.
+int res_clusters(const ResPlan& p, int units, int cus) { return std::max(1, std::min(units, cus / p.slabs)); }
+
 // Workgroups of one multi-unit launch (a multiple of 8): the tuned grid if
 // one is set, else one wavefront per work item, so the hardware dispatcher
 // hands the next item to whichever SIMD frees up first (items differ in cost:
@@ -1116,7 +1127,7 @@ struct ResRun {
 
 // Clears the exchange words and makes (v dt)^2, in stream order.
 int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom& g, const Sched& sc, const JobDesc& j,
-              const BatchLayout& L, const UnitDesc* units, const ResPlan& plan, int capacity, ResRun* run)
+              const BatchLayout& L, const UnitDesc* units, const ResPlan& plan, int cus, ResRun* run)
 {
     const int64_t n = (int64_t)nsample * g.ns;
     HIP_TRY(launch_zero(st, reinterpret_cast<float*>(L.halo), 2 * n * L.halo_stride + kResTickets));
@@ -1135,7 +1146,7 @@ int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geo
     a.vdt2_off = (int)(g.fe * sizeof(float));
     a.plan = plan;
     a.nunit = (int)n;
-    a.clusters = std::max(1, std::min((int)n, capacity / plan.slabs));
+    a.clusters = res_clusters(plan, (int)n, cus);
     return 0;
 }
 
@@ -1268,10 +1279,9 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     ResChoice rcho;
     rcho.ok = false;
     if (room) res_choose(g, nsample * g.ns, &rcho);
-    const int res_cap = rcho.ok ? std::min(res_capacity(g.lc), stream_cus(st)) : 0;
-    const bool resident_fits = res_cap > 0 && res_cap >= rcho.plan.slabs;
+    const int cus = res_cus(g, rcho, st);
     BatchLayout L;
-    if (phase != GPVI_PHASE_ADJOINT && (room = resident_fits)) {
+    if (phase != GPVI_PHASE_ADJOINT && (room = cus > 0)) {
         // (a workspace without the room keeps the launches: it may be sized for them)
         batch_layout(g, sc, nsample, true, true, nullptr, &L, model_only);
         room = L.bytes <= workspace_bytes;
@@ -1279,7 +1289,7 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     batch_layout(g, sc, nsample, true, room, nullptr, &L, model_only);
     if ((rc = check_workspace(workspace, workspace_bytes, L.bytes))) return rc;
     batch_layout(g, sc, nsample, true, room, (char*)workspace, &L, model_only);
-    const bool resident = room && resident_fits;
+    const bool resident = room && cus > 0;
     if (phase != GPVI_PHASE_ADJOINT) {
         if ((rc = job_setup(st, p, g, vel_inner, L.vel, L.vel_stride, L.wav, L.zero, nsample))) return rc;
     }
@@ -1346,7 +1356,7 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     }
     if (resident) {
         ResRun run;
-        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho.plan, res_cap, &run))) return rc;
+        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho.plan, cus, &run))) return rc;
         if ((rc = res_steps(st, &run, 0, run.total))) return rc;
         if (phase != GPVI_PHASE_FORWARD)
             HIP_TRY(launch_grad_reduce(st, L.gpriv, L.grad_stride, grad, g.ns, g.ni, nsample));
@@ -1393,6 +1403,25 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     if (phase != GPVI_PHASE_ADJOINT && misfit)
         HIP_TRY(launch_misfit(st, record_syn, record_obs, (int64_t)g.ns * g.nt * g.nr, nsample, L.partial, misfit));
     return 0;
+}
+
+int gpvi_fwi2d_resident_plan(const gpvi_fwi2d_params* p, int nsample, void* stream, int* slabs, int* clusters,
+                             int* steps)
+{
+    int rc = validate(p);
+    if (rc) return rc;
+    if (nsample < 1) return fail(GPVI_ERR_INVALID, "nsample=%d", nsample);
+    const Tuning tn = tuning();
+    Geom g;
+    make_geom(p, kDefaultVariant, 1, &g);   // (the plan depends on no launch shape)
+    ResChoice c;
+    c.ok = false;
+    if (tn.variant < 0 && tn.grid == 0 && tn.tb == 1) res_choose(g, nsample * g.ns, &c);
+    const int cus = res_cus(g, c, (hipStream_t)stream);
+    if (slabs) *slabs = cus ? c.plan.slabs : 0;
+    if (clusters) *clusters = cus ? res_clusters(c.plan, nsample * g.ns, cus) : 0;
+    if (steps) *steps = cus ? kResChunk : 0;
+    return cus ? 1 : 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1685,10 +1714,10 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
     ResChoice rcho;
     rcho.ok = false;
     if (e->resident) res_choose(jb.g, jb.nunit, &rcho);
-    const int res_cap = rcho.ok ? std::min(res_capacity(jb.g.lc), stream_cus(e->stream)) : 0;
+    const int cus = res_cus(jb.g, rcho, e->stream);
     batch_layout(jb.g, jb.sc, nsample, false, true, nullptr, &jb.L);
     // (a workspace without the room for the exchange words keeps the launches)
-    jb.resident = rcho.ok && res_cap >= rcho.plan.slabs && jb.L.bytes <= workspace_bytes;
+    jb.resident = cus > 0 && jb.L.bytes <= workspace_bytes;
     batch_layout(jb.g, jb.sc, nsample, false, jb.resident, nullptr, &jb.L);
     if ((rc = check_workspace(workspace, workspace_bytes, jb.L.bytes))) return rc;
     batch_layout(jb.g, jb.sc, nsample, false, jb.resident, (char*)workspace, &jb.L);
@@ -1717,7 +1746,7 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
         return fail(GPVI_ERR_CAPACITY, "step counter at %lld: let the engine drain before submitting", e->gstep);
     }
     if (jb.resident && (rc = res_begin(e->stream, p, nsample, jb.g, jb.sc, jb.j, jb.L, e->units + first, rcho.plan,
-                                       res_cap, &jb.run))) {
+                                       cus, &jb.run))) {
         engine_free_slots(e, first, jb.nunit);
         (void)hipEventDestroy(jb.done);
         return rc;
@@ -1844,6 +1873,14 @@ int gpvi_engine_cancel(gpvi_engine* e, long long job_id)
 }
 
 int gpvi_engine_active_jobs(gpvi_engine* e) { return e ? (int)e->active.size() : 0; }
+
+int gpvi_engine_resident_jobs(gpvi_engine* e)
+{
+    if (!e) return 0;
+    int n = 0;
+    for (const auto& jb : e->active) n += jb.res_now ? 1 : 0;
+    return n;
+}
 
 int gpvi_engine_active_units(gpvi_engine* e)
 {

@@ -131,6 +131,10 @@ class Engine:
     def active_units(self) -> int:
         return _lib.load().gpvi_engine_active_units(self._h)
 
+    def resident_jobs(self) -> int:
+        """Active jobs whose fields stayed on the chip in the last advance."""
+        return _lib.load().gpvi_engine_resident_jobs(self._h)
+
     def pending_steps(self) -> int:
         return _lib.load().gpvi_engine_pending_steps(self._h)
 

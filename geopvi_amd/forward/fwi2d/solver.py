@@ -80,6 +80,18 @@ def model_workspace_bytes(params: FWIParams, nsample: int) -> int:
     return int(n)
 
 
+def resident_plan(params: FWIParams, nsample: int, device=None) -> Optional[dict]:
+    """What a batched evaluation on the device's current stream does with the
+    launch shape set now: None where every step is a launch, else (the fields
+    stay on the chip) the workgroups of a unit ("slabs"), the units advanced
+    at a time ("clusters") and the time steps of a launch ("steps")."""
+    c, pc = _params_ptr(params)
+    slabs, clusters, steps = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    taken = _lib.check(_lib.load().gpvi_fwi2d_resident_plan(pc, int(nsample), _stream(device), ctypes.byref(slabs),
+                                                            ctypes.byref(clusters), ctypes.byref(steps)))
+    return {"slabs": slabs.value, "clusters": clusters.value, "steps": steps.value} if taken else None
+
+
 def schedule(params: FWIParams, ckpt_interval: int = 0, steps_per_launch: int = 1) -> dict:
     """Adjoint schedule and launch counts of a batched evaluation.
 

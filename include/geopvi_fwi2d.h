@@ -140,9 +140,19 @@ int gpvi_fwi2d_batch_static(const gpvi_fwi2d_params *p, int nsample, const float
                             const float *record_obs, float *record_syn, float *grad, double *misfit, int run_fwi,
                             int ckpt_interval, void *stream);
 
+/* Whether gpvi_fwi2d_batch of these parameters would keep the fields on the
+ * chip (1; given a workspace of full size) or launch every step (0), with the
+ * launch shape set now, on this stream.  If it would: the workgroups of one
+ * unit, the groups of them in a launch (each advances one unit at a time) and
+ * the time steps of a launch, at most.  The three may be NULL (0 if not). */
+int gpvi_fwi2d_resident_plan(const gpvi_fwi2d_params *p, int nsample, void *stream, int *slabs, int *clusters,
+                             int *steps);
+
 /* Launch shape of the multi-unit step: tile variant (0..5: rows per strip
- * segment; -1, the default: chosen per batched call, the longest segments
- * that still give each lane at least one resident grid of work items),
+ * segment; -1, the default: with grid 0 and one step per launch the fields
+ * stay on the chip where that is faster (gpvi_fwi2d_resident_plan), else the
+ * segments are chosen per batched call, the longest that still give each lane
+ * at least three quarters of a resident grid of work items),
  * persistent grid (a multiple of 8; 0 = one wavefront per work item) and
  * steps per graph segment.  Process-wide; the autotuner sets them.  The
  * workspace sizes do not depend on the variant. */
@@ -192,6 +202,9 @@ int gpvi_engine_release(gpvi_engine *e, long long job_id);
 int gpvi_engine_cancel(gpvi_engine *e, long long job_id);
 int gpvi_engine_active_jobs(gpvi_engine *e);
 int gpvi_engine_active_units(gpvi_engine *e);
+/* Active jobs whose fields stayed on the chip in the last advance (a few jobs
+ * do, one after the other; many share one launch per step). */
+int gpvi_engine_resident_jobs(gpvi_engine *e);
 /* Steps each active job still needs (maximum over jobs). */
 int gpvi_engine_pending_steps(gpvi_engine *e);
 int gpvi_engine_sync(gpvi_engine *e);
