@@ -342,7 +342,6 @@ Sched make_sched(const Geom& g, int ckpt_req)
 // and 29, 80 of them 54 and 51; 16 of 328x928 26 and 27, 30 of them 49 and 34.
 constexpr double kResRoundUs = 1.06, kResRowUs = 0.072, kResHaloRows = 2.2;
 constexpr double kStepUs = 12.0, kStepUsPerMpoint = 3.0, kStepUsPerLc = 0.09;
-constexpr int kResCus = 256;
 constexpr int kResTickets = 4096;    // launches between two clears
 constexpr int kResChunk = 256;       // time steps per launch
 
@@ -355,17 +354,15 @@ double step_launch_us(int lc, double points)
 {
     return kStepUs + kStepUsPerMpoint * (1 + kStepUsPerLc * (lc - 4)) * 1e-6 * points;
 }
-// Slabs of a unit, at most.  Launches on different hardware queues run at the
-// same time, each with at most one cluster of which only some slabs have a CU:
-// with q queues, q (slabs - 1) < 256 always leaves one for a missing slab.
-int res_max_slabs()
+// Hardware queues whose launches may run at once (the runtime's default is 4
+// per process; 8 leaves room for a second process).
+int res_queues()
 {
-    static const int most = [] {
+    static const int queues = [] {
         const char* e = std::getenv("GPU_MAX_HW_QUEUES");
-        const int q = std::max(8, e ? std::atoi(e) : 0);
-        return std::max(1, std::min(kResMaxSlabs, kResCus / q));
+        return std::max(8, e ? std::atoi(e) : 0);
     }();
-    return most;
+    return queues;
 }
 std::mutex g_res_mu;
 std::map<std::tuple<int, int, int, int, int>, ResChoice> g_res_plans;
@@ -383,7 +380,7 @@ void res_choose(const Geom& g, int units, ResChoice* out)
         return;
     }
     const ResGeom rg{g.ntx, g.ntz, g.lc, g.pml};
-    const double best = res_select_plan(rg, units, kResCus, res_max_slabs(), &out->plan);
+    const double best = res_select_plan(rg, units, kResCus, res_slab_limit(res_queues()), &out->plan);
     out->ok = best >= 0;
     if (out->ok) {
         const int n = out->plan.slabs;
@@ -578,7 +575,7 @@ int res_cus(const Geom& g, const ResChoice& c, hipStream_t st)
 {
     if (!c.ok) return 0;
     const int cus = std::min(res_capacity(g.lc), stream_cus(st));
-    return cus >= c.plan.slabs ? cus : 0;
+    return res_admits(c.plan.slabs, res_queues(), cus) ? cus : 0;
 }
 
 // Groups of workgroups of a launch, one group per unit at a time.

@@ -34,6 +34,7 @@ constexpr int kResZBlock = 2;        // band rows of a strip computed together
 constexpr int kResBandSlabs = 3;     // slabs the z band of one edge may span
 constexpr int kResTables = kResBandSlabs + 1;
 constexpr int kResMaxSlabs = 32;
+constexpr int kResCus = 256;         // CUs that plans and their times are made for
 constexpr int kResLdsBytes = 160 * 1024;
 constexpr int kResLdsFront = 16 + 2 * kResWaves * kResItems + 32;   // words before the first buffer: ticket, items, taper
 constexpr int kResLdsBack = 16;      // floats after the last one
@@ -493,6 +494,20 @@ inline double res_make_plan(const ResGeom& g, int slabs, ResPlan* p, double limi
     p->lds_bytes = res_lds_bytes(g.ntx, tallest, p->hr);
     return p->lds_bytes <= kResLdsBytes ? cost : -1;
 }
+
+// Which plans may run.  Launches on different hardware queues run at the same
+// time, each with at most one cluster of which only some slabs have a CU: with
+// queues (slabs - 1) < cus one is always left for a missing slab.  A stream or
+// device with fewer CUs than a plan is made for keeps the step launches: the
+// plan's time does not hold there, and streams with a CU mask have hardware
+// queues of their own beside the counted ones.
+inline bool res_admits(int slabs, int queues, int cus)
+{
+    return slabs >= 1 && cus >= kResCus && (long long)queues * (slabs - 1) < cus;
+}
+
+// The most slabs that are admitted on a whole chip.
+inline int res_slab_limit(int queues) { return std::min(kResMaxSlabs, (kResCus - 1) / std::max(1, queues) + 1); }
 
 // Rounds a launch takes over `units` units in `slabs` slabs each on `cus` CUs.
 inline double res_rounds(int units, int slabs, int cus)

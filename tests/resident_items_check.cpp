@@ -1,5 +1,6 @@
 // Checks of the row ranges that the resident steps' wavefronts take from a
-// plan (fwi2d_resident.h), as the kernel reads them: packed and unpacked.
+// plan (fwi2d_resident.h), as the kernel reads them: packed and unpacked; and
+// the rule of which plans may run.
 #include <vector>
 
 #include "fwi2d_resident.h"
@@ -54,3 +55,6 @@ extern "C" int resident_items_of_choice(int ntx, int ntz, int lc, int pml, int u
     if (res_select_plan(ResGeom{ntx, ntz, lc, pml}, units, 256, kResMaxSlabs, &p) < 0) return 0;
     return check_plan(p, ntx, ntz);
 }
+
+extern "C" int resident_admits(int slabs, int queues, int cus) { return res_admits(slabs, queues, cus) ? 1 : 0; }
+extern "C" int resident_slab_limit(int queues) { return res_slab_limit(queues); }

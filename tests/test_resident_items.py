@@ -37,3 +37,18 @@ def test_items_lie_in_their_slabs(lib, lc, pml0):
                 assert r >= 0, f"{nz}x{nx} lc {lc} pml0 {pml0} {slabs} slabs: fault {r}"
                 made += r
     assert made > 0
+
+
+def test_plans_that_may_run(lib):
+    """Every admitted plan leaves a CU for a missing slab whatever the launches
+    on the other queues hold; fewer CUs than a plan is made for are refused."""
+    for queues in (1, 4, 8, 10, 16, 31, 32, 300):
+        most = lib.resident_slab_limit(queues)
+        assert 1 <= most <= 32 and lib.resident_admits(most, queues, 256)
+        assert most == 32 or not lib.resident_admits(most + 1, queues, 256)
+        for slabs in range(1, 33):
+            held = queues * (slabs - 1)          # CUs of the launches' partial clusters, at most
+            assert bool(lib.resident_admits(slabs, queues, 256)) == (held < 256)
+    for cus in (0, 1, 32, 40, 63, 128, 255):     # a CU mask, a partition of the device
+        for slabs in (1, 2, 20, 32):
+            assert not lib.resident_admits(slabs, 8, cus)
