@@ -342,8 +342,14 @@ Sched make_sched(const Geom& g, int ckpt_req)
 // and 29, 80 of them 54 and 51; 16 of 328x928 26 and 27, 30 of them 49 and 34.
 constexpr double kResRoundUs = 1.06, kResRowUs = 0.072, kResHaloRows = 2.2;
 constexpr double kStepUs = 12.0, kStepUsPerMpoint = 3.0, kStepUsPerLc = 0.09;
-constexpr int kResTickets = 4096;    // launches between two clears
+constexpr int kResTickets = 4096;    // words for tickets and arrivals between two clears
 constexpr int kResChunk = 256;       // time steps per launch
+constexpr int kResGroup = 4;         // launches before clusters that gave up catch up
+// How long a cluster waits for its workgroups: what is between them and a CU
+// (other launches, this one's complete clusters) takes some launches' time.
+// Too short costs steps through memory, too long that much time wherever
+// launches of several processes hold CUs for each other.
+constexpr double kResJoinUs = 50e3, kResJoinLaunches = 4;
 
 struct ResChoice {
     bool ok;
@@ -1118,21 +1124,25 @@ struct ResRun {
     ResArgs a;
     UnitDesc sd;          // what decode_step reads
     unsigned* tickets;
-    int used;             // launches since the tickets were cleared
+    int used;             // words taken since the tickets were cleared
+    int behind;           // launches since units of clusters that gave up caught up
+    double step_us;       // modelled time of a step
     int lc, s_off, total;
 };
 
 // Clears the exchange words and makes (v dt)^2, in stream order.
 int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom& g, const Sched& sc, const JobDesc& j,
-              const BatchLayout& L, const UnitDesc* units, const ResPlan& plan, int cus, ResRun* run)
+              const BatchLayout& L, const UnitDesc* units, const ResChoice& choice, int cus, ResRun* run)
 {
+    const ResPlan& plan = choice.plan;
     const int64_t n = (int64_t)nsample * g.ns;
     HIP_TRY(launch_zero(st, reinterpret_cast<float*>(L.halo), 2 * n * L.halo_stride + kResTickets));
     HIP_TRY(launch_vdt2(st, L.vel, L.vel + g.fe, p->dt, (int64_t)g.ntz * g.pitch, L.vel_stride, nsample));
     std::memset(&run->sd, 0, sizeof run->sd);
     run->sd.nt = g.nt; run->sd.tb = 1; run->sd.nseg = sc.nseg; run->sd.ckpt = sc.ckpt; run->sd.last_len = sc.last_len;
     run->tickets = reinterpret_cast<unsigned*>(L.halo + n * L.halo_stride);
-    run->used = 0;
+    run->used = run->behind = 0;
+    run->step_us = choice.res_us;
     run->lc = g.lc;
     run->s_off = j.s_off;
     run->total = j.total;
@@ -1147,6 +1157,17 @@ int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geo
     return 0;
 }
 
+// The units whose cluster gave up in a launch since the last call catch up.
+// Due behind kResGroup launches, before anything else reads the fields or the
+// outputs, and before the tickets are cleared.
+int res_catch_up(hipStream_t st, ResRun* run)
+{
+    if (run->behind == 0) return 0;
+    run->behind = 0;
+    HIP_TRY(launch_resident_redo(st, run->lc, run->a, run->a.s0 + run->a.n));
+    return 0;
+}
+
 // Steps [s, end) with the fields on the chip: launches of up to kResChunk
 // steps, each within one pass (forward, a segment's recompute, an adjoint
 // stretch).
@@ -1154,6 +1175,14 @@ int res_steps(hipStream_t st, ResRun* run, int s, int end)
 {
     auto at = [&](int i) { return decode_step(run->sd, i + run->s_off); };
     end = std::min(end, run->total);
+    ResArgs& a = run->a;
+    const bool join = a.plan.slabs > 1;
+    const int counts = join ? a.clusters : 0;
+    // (tests: a limit in us, and with one below 0 every cluster of several workgroups gives up)
+    const char* limit = std::getenv("GPVI_RES_JOIN_US");
+    const double limit_us = limit && *limit ? std::atof(limit) : 0;
+    a.join.slabs = join ? (unsigned)a.plan.slabs : 0;
+    a.join.want = (unsigned)a.plan.slabs + (limit_us < 0 ? 1 : 0);
     while (s < end) {
         const StepInfo first = at(s);
         int n = 1;
@@ -1165,15 +1194,27 @@ int res_steps(hipStream_t st, ResRun* run, int s, int end)
             }
             ++n;
         }
-        if (run->used == kResTickets) {
+        if (run->used + 1 + 2 * counts > kResTickets) {
+            if (const int rc = res_catch_up(st, run)) return rc;
             HIP_TRY(launch_zero(st, reinterpret_cast<float*>(run->tickets), kResTickets));
             run->used = 0;
         }
-        run->a.ticket = run->tickets + run->used++;
-        run->a.s0 = s + run->s_off;
-        run->a.n = n;
-        HIP_TRY(launch_resident(st, run->lc, first.mode == kAdj, run->a));
+        if (run->behind == 0) {
+            a.join.gone = run->tickets + run->used;
+            run->used += counts;
+        }
+        a.ticket = run->tickets + run->used;
+        a.join.arrived = a.ticket + 1;
+        run->used += 1 + counts;
+        a.s0 = s + run->s_off;
+        a.join.step = (unsigned)a.s0;
+        a.n = n;
+        const double us = limit && *limit ? limit_us : kResJoinUs + kResJoinLaunches * n * run->step_us;
+        a.join.ticks = (unsigned long long)(100.0 * std::max(0.0, us));
+        HIP_TRY(launch_resident(st, run->lc, first.mode == kAdj, a));
         s += n;
+        if (join && ++run->behind == kResGroup)
+            if (const int rc = res_catch_up(st, run)) return rc;
     }
     return 0;
 }
@@ -1353,8 +1394,8 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     }
     if (resident) {
         ResRun run;
-        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho.plan, cus, &run))) return rc;
-        if ((rc = res_steps(st, &run, 0, run.total))) return rc;
+        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho, cus, &run))) return rc;
+        if ((rc = res_steps(st, &run, 0, run.total)) || (rc = res_catch_up(st, &run))) return rc;
         if (phase != GPVI_PHASE_FORWARD)
             HIP_TRY(launch_grad_reduce(st, L.gpriv, L.grad_stride, grad, g.ns, g.ni, nsample));
         if (phase != GPVI_PHASE_ADJOINT && misfit)
@@ -1580,7 +1621,7 @@ int engine_rebuild(gpvi_engine* e)
 // launches and take 13.8 ms; a stream at half load 46 and 27 ms (median).
 // Many small jobs share a launch better: at saturation the choice stays with
 // the launches (317 samples/s, 315 without resident steps).
-void engine_pick(gpvi_engine* e)
+int engine_pick(gpvi_engine* e)
 {
     double all = 0, rest = 0, res = 0;   // step launches of all jobs, of the others; resident steps
     int lc_all = 4, lc_rest = 4;
@@ -1597,17 +1638,21 @@ void engine_pick(gpvi_engine* e)
             others = true;
         }
     }
+    int rc = 0;
     const bool use = res + (others ? step_launch_us(lc_rest, rest) : 0) < step_launch_us(lc_all, all);
     for (auto& jb : e->active) {
         const bool now = use && jb.resident;
         if (now != jb.res_now) e->dirty = true;
+        if (!now && !rc) rc = res_catch_up(e->stream, &jb.run);
         jb.res_now = now;
     }
+    return rc;
 }
 
 int engine_finalize(gpvi_engine* e, EngineJob& jb)
 {
     if (!jb.cancelled) {
+        if (const int rc = res_catch_up(e->stream, &jb.run)) return rc;
         HIP_TRY(launch_grad_reduce(e->stream, jb.L.gpriv, jb.L.grad_stride, jb.grad, jb.g.ns, jb.g.ni,
                                    jb.j.nsample));
         if (jb.misfit)
@@ -1719,6 +1764,7 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
     if ((rc = check_workspace(workspace, workspace_bytes, jb.L.bytes))) return rc;
     batch_layout(jb.g, jb.sc, nsample, false, jb.resident, (char*)workspace, &jb.L);
     jb.res_now = false;
+    jb.run.behind = 0;
     jb.res_us = rcho.ok ? rcho.res_us : 0;
     int tiles_now = 0;
     for (const auto& a : e->active) tiles_now += a.nunit * a.g.tpu;
@@ -1742,8 +1788,8 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
         (void)hipEventDestroy(jb.done);
         return fail(GPVI_ERR_CAPACITY, "step counter at %lld: let the engine drain before submitting", e->gstep);
     }
-    if (jb.resident && (rc = res_begin(e->stream, p, nsample, jb.g, jb.sc, jb.j, jb.L, e->units + first, rcho.plan,
-                                       cus, &jb.run))) {
+    if (jb.resident && (rc = res_begin(e->stream, p, nsample, jb.g, jb.sc, jb.j, jb.L, e->units + first, rcho, cus,
+                                       &jb.run))) {
         engine_free_slots(e, first, jb.nunit);
         (void)hipEventDestroy(jb.done);
         return rc;
@@ -1768,7 +1814,7 @@ int gpvi_engine_advance(gpvi_engine* e, int nsteps)
     if (!e) return fail(GPVI_ERR_INVALID, "NULL engine");
     TraceRange tr("gpvi_engine_advance %zu jobs", e->active.size());
     int rc;
-    if (nsteps > 0) engine_pick(e);
+    if (nsteps > 0 && (rc = engine_pick(e))) return rc;
     if (e->dirty && (rc = engine_rebuild(e))) return rc;
     if (e->active.empty() || nsteps <= 0) return 0;
     int mask = 0;

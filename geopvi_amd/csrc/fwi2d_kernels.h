@@ -50,6 +50,7 @@ void variant_tile(int variant, int* tx, int* tz);
 constexpr int kNumVariants = 6;
 constexpr int kStripWidth = 64;
 constexpr int kMultiThreads = 256;   // workgroup of the multi-unit step (4 independent waves)
+constexpr int kRedoThreads = 512;    // workgroup that advances one unit alone
 constexpr int kSingleThreads = 64;   // workgroup of the single-unit step (1 wave)
 
 hipError_t launch_step_single(int variant, int lc, int grid, hipStream_t st, const UnitDesc& u, int s);
@@ -69,10 +70,18 @@ int misfit_blocks(int64_t len);
 
 // Resident steps (fwi2d_resident.hip): `n` macro steps of one pass from macro
 // step s0 for every unit of the table, fields on the chip.
+struct ResJoin {
+    unsigned* arrived;          // [c]: workgroups of cluster c that arrived in this launch
+    unsigned* gone;             // [c]: 1 + the macro step at which cluster c gave up (0: it did not)
+    unsigned long long ticks;   // of 100 MHz that a workgroup waits for its cluster
+    unsigned slabs, want;       // workgroups of a cluster (0: one each, nothing to wait for); those that must arrive
+    unsigned step;              // s0
+};
 struct ResArgs {
     const UnitDesc* units;
     unsigned long long* halo;   // halo_stride words per unit, zero before the call's first launch
     unsigned* ticket;           // zero before every launch
+    ResJoin join;
     int64_t halo_stride;
     int vdt2_off;               // bytes from a sample's padded velocities to its (v dt)^2
     int s0, n;
@@ -80,6 +89,9 @@ struct ResArgs {
     ResPlan plan;
 };
 hipError_t launch_resident(hipStream_t st, int lc, bool adjoint, const ResArgs& a);
+// Behind resident launches with the same units, clusters and `gone` words: the
+// units of clusters that gave up advance to macro step `end` through memory.
+hipError_t launch_resident_redo(hipStream_t st, int lc, const ResArgs& a, int end);
 hipError_t launch_vdt2(hipStream_t st, const float* vel, float* out, float dt, int64_t n, int64_t stride, int nsample);
 int resident_capacity(int lc);
 

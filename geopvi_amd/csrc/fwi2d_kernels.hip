@@ -60,6 +60,29 @@ __global__ __launch_bounds__(NTH) __attribute__((amdgpu_waves_per_eu(TB == 1 && 
     }
 }
 
+// Advances the units whose cluster gave up in the resident launches before
+// this one (see resident_kernel) to macro step `end`: a workgroup per unit goes
+// through the unit's work items step by step.  Nothing here waits for another
+// workgroup.  The barrier between two steps is enough, as a workgroup's stores
+// and loads share one L1.  Nearly always a look at a word.
+template <int LC, int NTH>
+__global__ __launch_bounds__(NTH) void resident_redo_kernel(const UnitDesc* __restrict__ units,
+                                                            const unsigned* __restrict__ gone, int clusters, int end)
+{
+    constexpr int NW = NTH / 64;
+    __shared__ float rows[NW][wave_lds_floats(LC, 1)];
+    const int ui = blockIdx.x;
+    const unsigned from = gone[ui % clusters];
+    if (from == 0) return;   // (uniform)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const UnitDesc& u = units[ui];
+    const int items = 2 * u.band_tz + u.tiles_x * u.tiles_z;
+    for (int s = (int)from - 1; s < end; ++s) {
+        for (int t = wave; t < items; t += NW) process_item<LC, 1>(u, s, t, rows[wave]);
+        __syncthreads();
+    }
+}
+
 __global__ void advance_kernel(StepCtl* ctl, int n)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) ctl->step = ctl->step + n;
@@ -330,6 +353,25 @@ int multi_step_capacity(int lc, int tb)
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     return nb * cus;
+}
+
+template <int LC>
+static hipError_t launch_resident_redo_lc(hipStream_t st, const ResArgs& a, int end)
+{
+    hipLaunchKernelGGL((resident_redo_kernel<LC, kRedoThreads>), dim3(a.nunit), dim3(kRedoThreads), 0, st, a.units,
+                       a.join.gone, a.clusters, end);
+    return hipGetLastError();
+}
+
+hipError_t launch_resident_redo(hipStream_t st, int lc, const ResArgs& a, int end)
+{
+    switch (lc) {
+    case 4: return launch_resident_redo_lc<4>(st, a, end);
+    case 5: return launch_resident_redo_lc<5>(st, a, end);
+    case 6: return launch_resident_redo_lc<6>(st, a, end);
+    case 7: return launch_resident_redo_lc<7>(st, a, end);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 hipError_t launch_advance(hipStream_t st, StepCtl* ctl, int n)

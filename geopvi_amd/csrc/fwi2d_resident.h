@@ -36,6 +36,7 @@ constexpr int kResTables = kResBandSlabs + 1;
 constexpr int kResMaxSlabs = 32;
 constexpr int kResCus = 256;         // CUs that plans and their times are made for
 constexpr int kResLdsBytes = 160 * 1024;
+constexpr unsigned kResGone = 0x80000000u;   // in a cluster's count of arrived workgroups: given up
 constexpr int kResLdsFront = 16 + 2 * kResWaves * kResItems + 32;   // words before the first buffer: ticket, items, taper
 constexpr int kResLdsBack = 16;      // floats after the last one
 
