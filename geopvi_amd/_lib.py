@@ -20,6 +20,7 @@ GPVI_FLAG_NO_STORE = 2
 GPVI_FLAG_ONE_STREAM = 4
 GPVI_ERR_HIP = -5  # HIP runtime failure (include/geopvi_fwi2d.h)
 GPVI_ERR_CAPACITY = -7  # engine unit/tile tables full (include/geopvi_fwi2d.h)
+GPVI_ERR_TIMEOUT = -9  # a wait between workgroups ran out (include/geopvi_fwi2d.h)
 
 # Every exported symbol and its ctypes signature: (restype, argtypes).
 _P = ctypes.POINTER(CParams)
@@ -38,6 +39,7 @@ SIGNATURES = {
     "gpvi_fwi2d_model_workspace_bytes": (_sz, [_P, _i]),
     "gpvi_fwi2d_batch": (_i, [_P, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _sz, _vp]),
     "gpvi_fwi2d_batch_static": (_i, [_P, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _vp]),
+    "gpvi_fwi2d_wait_status": (_i, [_vp]),
     "gpvi_fwi2d_resident_plan": (_i, [_P, _i, _vp] + [ctypes.POINTER(_i)] * 3),
     "gpvi_fwi2d_set_tuning": (_i, [_i, _i, _i]),
     "gpvi_fwi2d_get_tuning": (_i, [ctypes.POINTER(_i)] * 3),

@@ -6,6 +6,7 @@
 #include <rocprofiler-sdk-roctx/roctx.h>
 
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <cstdarg>
@@ -344,12 +345,15 @@ constexpr double kResRoundUs = 1.06, kResRowUs = 0.072, kResHaloRows = 2.2;
 constexpr double kStepUs = 12.0, kStepUsPerMpoint = 3.0, kStepUsPerLc = 0.09;
 constexpr int kResTickets = 4096;    // words for tickets and arrivals between two clears
 constexpr int kResChunk = 256;       // time steps per launch
-constexpr int kResGroup = 4;         // launches before clusters that gave up catch up
+constexpr int kResCatchUp = 1024;    // time steps before clusters that gave up catch up
 // How long a cluster waits for its workgroups: what is between them and a CU
 // (other launches, this one's complete clusters) takes some launches' time.
 // Too short costs steps through memory, too long that much time wherever
 // launches of several processes hold CUs for each other.
 constexpr double kResJoinUs = 50e3, kResJoinLaunches = 4;
+// How long a wait for a neighbour's rows may take.  The whole cluster is on
+// CUs by then, so only a preempted process waits at all long.
+constexpr double kResWaitUs = 20e6;
 
 struct ResChoice {
     bool ok;
@@ -1119,20 +1123,66 @@ int layout_stamp_get(const void* ws, const gpvi_fwi2d_params* p, int nsample, in
     return 0;
 }
 
+// The word, one per device, in which a resident launch of a batched call whose
+// wait ran out leaves the call's number (engine jobs have words of their own).
+// Placed by the code-object loader; looked up once per device.
+static __device__ unsigned res_fault_word;
+constexpr int kMaxDevices = 64;
+std::atomic<unsigned> g_res_calls{0};
+// Per thread and device: the first call that the thread numbered there, and the
+// last failed one it was told of.
+struct FaultSeen {
+    unsigned first, told;
+};
+thread_local FaultSeen g_fault_seen[kMaxDevices] = {};
+
+int res_fault(unsigned** word, int* device)
+{
+    static std::mutex mu;
+    static unsigned* words[kMaxDevices] = {};
+    HIP_TRY(hipGetDevice(device));
+    if (*device < 0 || *device >= kMaxDevices) return fail(GPVI_ERR_HIP, "device %d out of range", *device);
+    std::lock_guard<std::mutex> lk(mu);
+    if (!words[*device]) {
+        void* p = nullptr;
+        HIP_TRY(hipGetSymbolAddress(&p, HIP_SYMBOL(res_fault_word)));
+        words[*device] = (unsigned*)p;
+    }
+    *word = words[*device];
+    return 0;
+}
+
+// Behind a synchronisation: whether a wait ran out in a call of this thread.
+int res_fault_status()
+{
+    unsigned* word;
+    int dev;
+    if (const int rc = res_fault(&word, &dev)) return rc;
+    FaultSeen& f = g_fault_seen[dev];
+    if (f.first == 0) return 0;   // no such call
+    unsigned id = 0;
+    HIP_TRY(hipMemcpy(&id, word, sizeof id, hipMemcpyDeviceToHost));
+    if (id == f.told || id - f.first >= 0x80000000u) return 0;   // (numbers may wrap)
+    f.told = id;
+    return fail(GPVI_ERR_TIMEOUT, "a wait between workgroups ran out in a batched call (%.0f s): its outputs are invalid",
+                kResWaitUs * 1e-6);
+}
+
 // The resident steps of a batch or an engine job.
 struct ResRun {
     ResArgs a;
     UnitDesc sd;          // what decode_step reads
     unsigned* tickets;
     int used;             // words taken since the tickets were cleared
-    int behind;           // launches since units of clusters that gave up caught up
+    int behind;           // steps since units of clusters that gave up caught up
     double step_us;       // modelled time of a step
     int lc, s_off, total;
 };
 
 // Clears the exchange words and makes (v dt)^2, in stream order.
 int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geom& g, const Sched& sc, const JobDesc& j,
-              const BatchLayout& L, const UnitDesc* units, const ResChoice& choice, int cus, ResRun* run)
+              const BatchLayout& L, const UnitDesc* units, const ResChoice& choice, int cus, unsigned* fault,
+              unsigned fault_id, ResRun* run)
 {
     const ResPlan& plan = choice.plan;
     const int64_t n = (int64_t)nsample * g.ns;
@@ -1154,11 +1204,16 @@ int res_begin(hipStream_t st, const gpvi_fwi2d_params* p, int nsample, const Geo
     a.plan = plan;
     a.nunit = (int)n;
     a.clusters = res_clusters(plan, (int)n, cus);
+    const char* limit = std::getenv("GPVI_RES_WAIT_US");   // (tests)
+    const double us = limit && *limit ? std::max(0.0, std::atof(limit)) : kResWaitUs;
+    a.wait = (unsigned)std::min(100.0 * us / 65536.0, 4e9);
+    a.fault = fault;
+    a.fault_id = fault_id;
     return 0;
 }
 
 // The units whose cluster gave up in a launch since the last call catch up.
-// Due behind kResGroup launches, before anything else reads the fields or the
+// Due behind kResCatchUp steps, before anything else reads the fields or the
 // outputs, and before the tickets are cleared.
 int res_catch_up(hipStream_t st, ResRun* run)
 {
@@ -1213,7 +1268,7 @@ int res_steps(hipStream_t st, ResRun* run, int s, int end)
         a.join.ticks = (unsigned long long)(100.0 * std::max(0.0, us));
         HIP_TRY(launch_resident(st, run->lc, first.mode == kAdj, a));
         s += n;
-        if (join && ++run->behind == kResGroup)
+        if (join && (run->behind += n) >= kResCatchUp)
             if (const int rc = res_catch_up(st, run)) return rc;
     }
     return 0;
@@ -1394,7 +1449,13 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     }
     if (resident) {
         ResRun run;
-        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho, cus, &run))) return rc;
+        unsigned* fault;
+        int dev;
+        if ((rc = res_fault(&fault, &dev))) return rc;
+        unsigned id = ++g_res_calls;
+        if (id == 0) id = ++g_res_calls;
+        if (g_fault_seen[dev].first == 0) g_fault_seen[dev].first = id;
+        if ((rc = res_begin(st, p, nsample, g, sc, j, L, L.units, rcho, cus, fault, id, &run))) return rc;
         if ((rc = res_steps(st, &run, 0, run.total)) || (rc = res_catch_up(st, &run))) return rc;
         if (phase != GPVI_PHASE_FORWARD)
             HIP_TRY(launch_grad_reduce(st, L.gpriv, L.grad_stride, grad, g.ns, g.ni, nsample));
@@ -1443,6 +1504,12 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params* p, int nsample, const float* vel_i
     return 0;
 }
 
+int gpvi_fwi2d_wait_status(void* stream)
+{
+    HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    return res_fault_status();
+}
+
 int gpvi_fwi2d_resident_plan(const gpvi_fwi2d_params* p, int nsample, void* stream, int* slabs, int* clusters,
                              int* steps)
 {
@@ -1476,7 +1543,6 @@ namespace {
 constexpr size_t kStaticScratchBytes = (size_t)GPVI_STATIC_SCRATCH_BYTES;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 
-constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
 void* g_scratch_ptr[kMaxDevices] = {};
 
@@ -1532,6 +1598,10 @@ int gpvi_fwi2d_batch_static(const gpvi_fwi2d_params* p, int nsample, const float
 
 namespace {
 
+// Jobs in flight or unreleased that may run resident steps, at most (further
+// ones take the launches).
+constexpr int kEngineFaults = 4096;
+
 struct EngineJob {
     long long id;
     Geom g;
@@ -1546,12 +1616,19 @@ struct EngineJob {
     const float* obs;
     hipEvent_t done;
     bool cancelled;
+    int fault;                // its word in the engine's `faults` (-1: none)
     bool resident, res_now;   // can run resident steps; runs them in this advance
     double res_us;            // modelled time of one
     ResRun run;
 };
 
 }  // namespace
+
+// A job whose last kernels are enqueued.
+struct EngineDone {
+    hipEvent_t event;
+    int fault;
+};
 
 struct gpvi_engine {
     hipStream_t stream;
@@ -1565,7 +1642,9 @@ struct gpvi_engine {
     long long next_id;
     bool dirty;
     std::vector<EngineJob> active;
-    std::map<long long, hipEvent_t> finished;
+    std::map<long long, EngineDone> finished;
+    unsigned* faults;               // host memory: set where a wait of a job ran out
+    std::vector<int> fault_free;    // words of `faults` that no job has
     std::vector<unsigned char> slot_used;
     std::vector<hipEvent_t> inflight;
 };
@@ -1688,13 +1767,16 @@ int gpvi_engine_create(void* stream, int max_units, int max_tiles, gpvi_engine**
     hipError_t err = hipMalloc((void**)&e->units, sizeof(UnitDesc) * (size_t)max_units);
     if (err == hipSuccess) err = hipMalloc((void**)&e->tiles, sizeof(TileRef) * (size_t)max_tiles);
     if (err == hipSuccess) err = hipMalloc((void**)&e->ctl, sizeof(StepCtl));
+    if (err == hipSuccess) err = hipHostMalloc((void**)&e->faults, sizeof(unsigned) * kEngineFaults, hipHostMallocDefault);
     if (err != hipSuccess) {
         if (e->units) (void)hipFree(e->units);
         if (e->tiles) (void)hipFree(e->tiles);
         if (e->ctl) (void)hipFree(e->ctl);
+        if (e->faults) (void)hipHostFree(e->faults);
         delete e;
         return fail(GPVI_ERR_HIP, "engine tables: %s", hipGetErrorString(err));
     }
+    for (int i = kEngineFaults; i-- > 0;) e->fault_free.push_back(i);
     *out = e;
     return 0;
 }
@@ -1714,7 +1796,7 @@ int gpvi_engine_destroy(gpvi_engine* e)
     (void)hipStreamSynchronize(e->stream);
     for (auto ev : e->inflight) (void)hipEventDestroy(ev);
     for (auto& jb : e->active) (void)hipEventDestroy(jb.done);
-    for (auto& kv : e->finished) (void)hipEventDestroy(kv.second);
+    for (auto& kv : e->finished) (void)hipEventDestroy(kv.second.event);
     {
         std::lock_guard<std::mutex> lk(g_graph_mu);
         for (auto it = g_graphs.begin(); it != g_graphs.end();) {
@@ -1729,6 +1811,7 @@ int gpvi_engine_destroy(gpvi_engine* e)
     (void)hipFree(e->units);
     (void)hipFree(e->tiles);
     (void)hipFree(e->ctl);
+    (void)hipHostFree(e->faults);
     delete e;
     return 0;
 }
@@ -1756,7 +1839,7 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
     ResChoice rcho;
     rcho.ok = false;
     if (e->resident) res_choose(jb.g, jb.nunit, &rcho);
-    const int cus = res_cus(jb.g, rcho, e->stream);
+    const int cus = e->fault_free.empty() ? 0 : res_cus(jb.g, rcho, e->stream);
     batch_layout(jb.g, jb.sc, nsample, false, true, nullptr, &jb.L);
     // (a workspace without the room for the exchange words keeps the launches)
     jb.resident = cus > 0 && jb.L.bytes <= workspace_bytes;
@@ -1788,8 +1871,15 @@ int gpvi_engine_submit(gpvi_engine* e, const gpvi_fwi2d_params* p, int nsample, 
         (void)hipEventDestroy(jb.done);
         return fail(GPVI_ERR_CAPACITY, "step counter at %lld: let the engine drain before submitting", e->gstep);
     }
+    jb.fault = -1;
+    if (jb.resident) {
+        jb.fault = e->fault_free.back();
+        e->fault_free.pop_back();
+        e->faults[jb.fault] = 0;
+    }
     if (jb.resident && (rc = res_begin(e->stream, p, nsample, jb.g, jb.sc, jb.j, jb.L, e->units + first, rcho, cus,
-                                       &jb.run))) {
+                                       e->faults + jb.fault, 1, &jb.run))) {
+        e->fault_free.push_back(jb.fault);
         engine_free_slots(e, first, jb.nunit);
         (void)hipEventDestroy(jb.done);
         return rc;
@@ -1860,7 +1950,7 @@ int gpvi_engine_advance(gpvi_engine* e, int nsteps)
                 roctxMarkA(msg);
             }
             engine_free_slots(e, jb.j.unit0, jb.nunit);
-            e->finished[jb.id] = jb.done;
+            e->finished[jb.id] = EngineDone{jb.done, jb.fault};
             e->active.erase(e->active.begin() + i);
             e->dirty = true;
             ++ncomplete;
@@ -1876,8 +1966,13 @@ int gpvi_engine_job_status(gpvi_engine* e, long long job_id)
     if (!e) return fail(GPVI_ERR_INVALID, "NULL engine");
     auto it = e->finished.find(job_id);
     if (it != e->finished.end()) {
-        hipError_t q = hipEventQuery(it->second);
-        if (q == hipSuccess) return 1;
+        hipError_t q = hipEventQuery(it->second.event);
+        if (q == hipSuccess) {
+            const int f = it->second.fault;
+            if (f < 0 || __atomic_load_n(e->faults + f, __ATOMIC_ACQUIRE) == 0) return 1;
+            return fail(GPVI_ERR_TIMEOUT, "job %lld: a wait between workgroups ran out (%.0f s): its outputs are invalid",
+                        job_id, kResWaitUs * 1e-6);
+        }
         if (q == hipErrorNotReady) return 0;
         return fail(GPVI_ERR_HIP, "hipEventQuery: %s", hipGetErrorString(q));
     }
@@ -1891,8 +1986,9 @@ int gpvi_engine_release(gpvi_engine* e, long long job_id)
     if (!e) return fail(GPVI_ERR_INVALID, "NULL engine");
     auto it = e->finished.find(job_id);
     if (it == e->finished.end()) return fail(GPVI_ERR_UNKNOWN_JOB, "job %lld is not finished", job_id);
-    HIP_TRY(hipEventSynchronize(it->second));
-    (void)hipEventDestroy(it->second);
+    HIP_TRY(hipEventSynchronize(it->second.event));
+    (void)hipEventDestroy(it->second.event);
+    if (it->second.fault >= 0) e->fault_free.push_back(it->second.fault);
     e->finished.erase(it);
     return 0;
 }
@@ -1907,7 +2003,7 @@ int gpvi_engine_cancel(gpvi_engine* e, long long job_id)
         int rc = engine_finalize(e, jb);  // records the event after all work already queued
         if (rc) return rc;
         engine_free_slots(e, jb.j.unit0, jb.nunit);
-        e->finished[jb.id] = jb.done;
+        e->finished[jb.id] = EngineDone{jb.done, jb.fault};
         e->active.erase(e->active.begin() + i);
         e->dirty = true;
         return 0;
@@ -1998,8 +2094,9 @@ static int compat_run(char input_file[200], float* vel_inner, float* record_syn,
     }
     if (!rc) {
         err = hipDeviceSynchronize();
-        if (err == hipSuccess) err = hipMemcpy(record_syn, d_syn, nrec * sizeof(float), hipMemcpyDeviceToHost);
-        if (err == hipSuccess && adjoint) err = hipMemcpy(grad, d_grad, ni * sizeof(float), hipMemcpyDeviceToHost);
+        if (err == hipSuccess) rc = res_fault_status();
+        if (err == hipSuccess && !rc) err = hipMemcpy(record_syn, d_syn, nrec * sizeof(float), hipMemcpyDeviceToHost);
+        if (err == hipSuccess && !rc && adjoint) err = hipMemcpy(grad, d_grad, ni * sizeof(float), hipMemcpyDeviceToHost);
         if (err != hipSuccess) rc = fail(GPVI_ERR_HIP, "fwi_2D: %s", hipGetErrorString(err));
     }
     (void)hipFree(d_vel); (void)hipFree(d_syn); (void)hipFree(d_obs); (void)hipFree(d_grad); (void)hipFree(d_mis);

@@ -81,12 +81,15 @@ struct ResArgs {
     const UnitDesc* units;
     unsigned long long* halo;   // halo_stride words per unit, zero before the call's first launch
     unsigned* ticket;           // zero before every launch
-    ResJoin join;
     int64_t halo_stride;
     int vdt2_off;               // bytes from a sample's padded velocities to its (v dt)^2
     int s0, n;
     int nunit, clusters;        // units of the table; groups of plan.slabs workgroups
     ResPlan plan;
+    ResJoin join;
+    unsigned wait;              // 2^16 ticks of 100 MHz that a wait for a neighbour's rows may take
+    unsigned* fault;            // set to fault_id where one ran out (the outputs are then NaN or wrong)
+    unsigned fault_id;
 };
 hipError_t launch_resident(hipStream_t st, int lc, bool adjoint, const ResArgs& a);
 // Behind resident launches with the same units, clusters and `gone` words: the

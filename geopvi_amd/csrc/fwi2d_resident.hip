@@ -24,8 +24,9 @@
 // (resident_redo_kernel).  A cluster advances units cluster, cluster + clusters,
 // ... one after the other (workgroups queued behind a full chip are bound to
 // an XCD early and leave others idle: 320 units of 228x428 took two rounds more).
-// Every wait is bounded in time (kResWaitTicks); past it the halo becomes NaN
-// and nothing waits any more.
+// The waits for a neighbour's rows are bounded in time too (ResArgs::wait,
+// though with the whole cluster on CUs they end by themselves); past it the
+// halo becomes NaN, nothing waits any more and ResArgs::fault is set.
 //
 // What bounds it: vector issue, and per step about 2 us of exchange (a word
 // takes 0.7 us to a workgroup of the same XCD and up to 1.2 us across), barrier
@@ -44,9 +45,17 @@
 namespace gpvi {
 
 typedef __attribute__((address_space(3))) float LdsF;
+typedef __attribute__((address_space(3))) unsigned LdsU;
 
-// 100 MHz ticks a workgroup waits for a neighbour before it gives up (20 s).
-constexpr unsigned long long kResWaitTicks = 2000000000ull;
+// The LDS begins with kResLdsFront words: these, the items, the taper.  (The
+// time limit and whether a wait ran out are read in rare cases only; in
+// registers they would cost the steps some.)
+enum ResFront : int { kFrontTicket = 0, kFrontWait = 1, kFrontFault = 2, kFrontItems = 16 };
+__device__ __forceinline__ LdsU* res_front()
+{
+    extern __shared__ __align__(16) float res_lds[];
+    return (LdsU*)(LdsF*)res_lds;
+}
 
 // The unit table is not written while a resident kernel runs: reads through
 // the constant address space stay scalar.
@@ -442,8 +451,12 @@ __device__ __forceinline__ void res_ask(ResRecv<LC>& r, const ResPoll& p, int P,
 }
 
 // Repeats the loads until every word carries this step's tag and stores the
-// rows at `dst`; false once the wait has run out (the rows are then NaN).
-template <int LC>
+// rows at `dst`; false once the wait has run out (the rows are then NaN).  A
+// forward kernel notes that in the LDS too, an adjoint one only in `alive`:
+// the same outcome, and the better register allocation of each (with the note,
+// 20 units of 228x428 take 1.5 % longer in all; without it 48 units of 138x278
+// take 2 % longer forward).
+template <int LC, bool ADJ>
 __device__ __forceinline__ bool res_await(ResRecv<LC>& r, const ResPoll& p, LdsF* dst, int P, unsigned tag, bool alive)
 {
     constexpr int HR = ResRecv<LC>::HR;
@@ -456,8 +469,9 @@ __device__ __forceinline__ bool res_await(ResRecv<LC>& r, const ResPoll& p, LdsF
     if (missing()) {
         const unsigned long long t0 = wall_clock64();
         do {
-            if (!alive || wall_clock64() - t0 > kResWaitTicks) {
+            if (!alive || wall_clock64() - t0 > (unsigned long long)res_front()[kFrontWait] << 16) {
                 alive = false;
+                if (!ADJ) res_front()[kFrontFault] = 1;
 #pragma unroll
                 for (int j = 0; j < HR; ++j) r.w[j] = ((unsigned long long)tag << 32) | 0x7fc00000ull;
             } else {
@@ -753,18 +767,19 @@ template <int LC, bool ADJ>
 __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
 {
     constexpr int HR = LC - 1 > 4 ? LC - 1 : 4;
-    extern __shared__ __align__(16) float res_lds[];
-    LdsF* const lds = (LdsF*)res_lds;
+    LdsF* const lds = (LdsF*)res_front();
     const ResPlan& pl = a.plan;
     if (threadIdx.x == 0) {
+        res_front()[kFrontWait] = a.wait;
+        res_front()[kFrontFault] = 0;
         unsigned t = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         // (expected not taken: the wait's code then stays out of the way of the steps' registers; forward
         // steps of 2 units of 52x68 take 4.58 us, 4.83 without the hint)
         if (__builtin_expect(a.join.slabs != 0, 0) && !res_join(a.join, t / a.join.slabs)) t = kResGone;   // past every unit
-        *(__attribute__((address_space(3))) unsigned*)lds = t;
+        res_front()[kFrontTicket] = t;
     }
     __syncthreads();
-    const unsigned ticket = __builtin_amdgcn_readfirstlane(*(__attribute__((address_space(3))) unsigned*)lds);
+    const unsigned ticket = __builtin_amdgcn_readfirstlane(res_front()[kFrontTicket]);
     // readfirstlane: what follows from the cluster and slab stays in scalar registers
     const int cluster = __builtin_amdgcn_readfirstlane((int)(ticket / (unsigned)pl.slabs));
     const int g = (int)ticket - cluster * pl.slabs;
@@ -820,8 +835,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
         }
     }
     // The wave's items, decoded, in LDS.
-    typedef __attribute__((address_space(3))) unsigned LdsU;
-    LdsU* const my_items = (LdsU*)lds + 16 + wave * 2 * kResItems;
+    LdsU* const my_items = (LdsU*)lds + kFrontItems + wave * 2 * kResItems;
     if (lane < kResItems) {
         const ResItem item = pl.item[sl.table][wave][lane];
         int start, dz, cnt;
@@ -831,7 +845,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
         my_items[2 * lane] = w0;
         my_items[2 * lane + 1] = w1;
     }
-    k.taper = lds + 16 + 2 * kResWaves * kResItems;
+    k.taper = lds + kFrontItems + 2 * kResWaves * kResItems;
     if (wave == 0 && lane < 32 && lane < u.pml0) k.taper[lane] = G(u.wtab)[lane];
     const bool two_phase = pl.two_phase[sl.table] != 0;
     // side blocks: column and row slot of this lane, left and right
@@ -947,7 +961,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
         if (recv) {
             if (poll.on) {
                 if (!asked) res_ask<LC>(rx, poll, P, s.tag);
-                alive = res_await<LC>(rx, poll, poll_dst, P, s.tag, alive);
+                alive = res_await<LC, ADJ>(rx, poll, poll_dst, P, s.tag, alive);
             }
 #pragma unroll
             for (int j = 1; j < kPolls; ++j) {
@@ -955,7 +969,7 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
                 const ResPoll p = poll_unit(j, hp, f0, &dst);
                 if (p.on) {
                     res_ask<LC>(rx, p, P, s.tag);
-                    alive = res_await<LC>(rx, p, dst, P, s.tag, alive);
+                    alive = res_await<LC, ADJ>(rx, p, dst, P, s.tag, alive);
                 }
             }
         }
@@ -977,6 +991,8 @@ __global__ __launch_bounds__(kResThreads) void resident_kernel(ResArgs a)
     }
     __syncthreads();   // the next unit reuses the buffers
     }
+    if (__builtin_expect(ADJ ? !alive : res_front()[kFrontFault] != 0, 0))
+        __hip_atomic_store(G(a.fault), a.fault_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // vdt2[m] = (vel[m] * dt)^2 for fields of n values, in and out fields each

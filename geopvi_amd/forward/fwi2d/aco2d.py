@@ -63,7 +63,9 @@ def fwi(vel, record_obs, paramfile="./input/input_param.txt", is_fwi=1, verbose=
     obs = torch.from_numpy(record_obs).to(dev)
     ckpt = solver.auto_ckpt_interval(params, 1, dev)
     syn, grad, _ = solver.fwi_batch(params, vel_f.view(1, -1), obs, run_fwi=int(is_fwi), ckpt_interval=ckpt)
-    return syn[0].cpu().numpy(), grad[0].cpu().numpy()
+    out = syn[0].cpu().numpy(), grad[0].cpu().numpy()
+    solver.check_waits(dev)
+    return out
 
 
 def forward(vel, dim=1, paramfile="./input/input_param.txt", verbose=0):
@@ -82,4 +84,5 @@ def forward(vel, dim=1, paramfile="./input/input_param.txt", verbose=0):
     syn = solver.forward_batch(params, torch.from_numpy(np.float32(vel)).to(dev).view(1, -1))
     out = np.zeros(dim, dtype=np.float32)
     out[: params.record_len] = syn[0].cpu().numpy()
+    solver.check_waits(dev)
     return out

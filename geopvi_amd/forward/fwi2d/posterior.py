@@ -123,6 +123,7 @@ class Posterior:
                                          ckpt_interval=self._ckpt(hi - lo))
             loss[lo:hi] = mis.cpu().numpy()
             grad[lo:hi] = -(g.cpu().numpy()[:, self.mask])
+            solver.check_waits(self.device)
         return loss, grad
 
     def fwi_parallel(self, x):

@@ -92,6 +92,14 @@ def resident_plan(params: FWIParams, nsample: int, device=None) -> Optional[dict
     return {"slabs": slabs.value, "clusters": clusters.value, "steps": steps.value} if taken else None
 
 
+def check_waits(device=None) -> None:
+    """Waits for the device's current stream and raises GpviError
+    (GPVI_ERR_TIMEOUT) if a wait between workgroups ran out in a batched call
+    of this thread since the last check: that call's outputs are invalid."""
+    with torch.cuda.device(device):
+        _lib.check(_lib.load().gpvi_fwi2d_wait_status(_stream(device)))
+
+
 def schedule(params: FWIParams, ckpt_interval: int = 0, steps_per_launch: int = 1) -> dict:
     """Adjoint schedule and launch counts of a batched evaluation.
 

@@ -482,9 +482,19 @@ class FWIServer:
                        ckpt_interval=res.extra.get("ckpt_interval"), chunks=res.extra.get("chunks", 1))
         self._log.write(json.dumps(rec) + "\n")
 
+    def _over(self, key):
+        """(whether the job is finished, the error of one whose outputs a
+        timed-out wait made invalid: it fails that request alone)."""
+        try:
+            return self.engines[key[0]].status(key[1]) == 1, None
+        except _lib.GpviError as exc:
+            if exc.code != _lib.GPVI_ERR_TIMEOUT:
+                raise
+            return True, _lib.GpviError(exc.code, exc.msg)
+
     def _reap(self):
-        done = [k for k in self._inflight if self.engines[k[0]].status(k[1]) == 1]
-        for k in done:
+        done = [(k, exc) for k in self._inflight for over, exc in [self._over(k)] if over]
+        for k, timeout in done:
             req = self._inflight.pop(k)
             self.engines[k[0]].release(k[1])
             self._units_in_use[k[0]] -= req.vel.shape[0] * req.params.ns
@@ -495,9 +505,9 @@ class FWIServer:
             self.arena.release(req.extra["arena_offset"], req.need)
             bad = self._nonfinite_rows(job.misfit)
             sp = req.split
-            if len(bad) and not req.future.done():
+            if (len(bad) or timeout) and not req.future.done():
                 lo = req.rows[0] if sp is not None else 0
-                exc = FloatingPointError(f"non-finite misfit for sample(s) {(bad + lo).tolist()}: unstable model "
+                exc = timeout or FloatingPointError(f"non-finite misfit for sample(s) {(bad + lo).tolist()}: unstable model "
                                          "or NaN/Inf in the observed data")
                 req.future.set_exception(exc)
                 self._write_log(req, None, f"failed: {exc}")

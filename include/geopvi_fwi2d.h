@@ -34,6 +34,7 @@ extern "C" {
 #define GPVI_ERR_WORKSPACE (-6)   /* workspace missing, too small or misaligned */
 #define GPVI_ERR_CAPACITY (-7)    /* engine unit/tile tables full */
 #define GPVI_ERR_UNKNOWN_JOB (-8) /* engine job id not known */
+#define GPVI_ERR_TIMEOUT (-9)     /* a wait between workgroups on the GPU ran out: the outputs are invalid */
 
 /* Phases of a batched evaluation. */
 #define GPVI_PHASE_ALL 0      /* forward + adjoint in one call */
@@ -148,6 +149,16 @@ int gpvi_fwi2d_batch_static(const gpvi_fwi2d_params *p, int nsample, const float
 int gpvi_fwi2d_resident_plan(const gpvi_fwi2d_params *p, int nsample, void *stream, int *slabs, int *clusters,
                              int *steps);
 
+/* Waits for the stream; then GPVI_ERR_TIMEOUT if a wait between workgroups ran
+ * out (20 s) in a batched call that this thread made on the current device,
+ * once for each such call, else 0.  With the fields on the chip a unit's
+ * workgroups wait for each other's edge rows.  They start only when all of
+ * them have a CU, so such a wait is long only where the process is held up;
+ * the outputs of the call (records, gradient, misfit) are then invalid.
+ * fwi_2D and forward_2D check it themselves, gpvi_engine_job_status reports it
+ * for engine jobs. */
+int gpvi_fwi2d_wait_status(void *stream);
+
 /* Launch shape of the multi-unit step: tile variant (0..5: rows per strip
  * segment; -1, the default: with grid 0 and one step per launch the fields
  * stay on the chip where that is faster (gpvi_fwi2d_resident_plan), else the
@@ -194,7 +205,8 @@ int gpvi_engine_submit(gpvi_engine *e, const gpvi_fwi2d_params *p, int nsample, 
  * segments); returns the number of jobs that completed (their finalising
  * kernels are enqueued). */
 int gpvi_engine_advance(gpvi_engine *e, int nsteps);
-/* 1 = outputs final, 0 = in flight, <0 = unknown id. */
+/* 1 = outputs final, 0 = in flight, GPVI_ERR_TIMEOUT = finished with invalid
+ * outputs (see gpvi_fwi2d_wait_status), other < 0 = unknown id or failure. */
 int gpvi_engine_job_status(gpvi_engine *e, long long job_id);
 /* Forget a finished job (frees its engine bookkeeping). */
 int gpvi_engine_release(gpvi_engine *e, long long job_id);
