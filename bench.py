@@ -4,15 +4,16 @@
 One "step" = one batched misfit+gradient evaluation of the c1 workload:
 16 velocity samples (mean-field Gaussian, std 50 m/s around the smoothed
 true model) x 20 shots on a 200x400 grid (228x428 padded), 200 receivers,
-8 Hz Ricker, dt = 1 ms, 2000 steps, nt_interval = 2, fp32, every
-(sample, shot) unit advanced by each step launch, replayed as HIP graph
-segments.  Inputs (models, observed data) are resident in HBM before the
+8 Hz Ricker, dt = 1 ms, 2000 steps, nt_interval = 2, fp32, with the fields
+on the chip or every (sample, shot) unit advanced by each step launch,
+replayed as HIP graph segments, whichever the autotuner finds faster.  Inputs (models, observed data) are resident in HBM before the
 timed region.  The launch shape is chosen by the autotuner (untimed).
 
 Printed (one JSON line): batched samples/s (``value``), the plain
 one-sample-per-launch GPU solver's samples/s on the same workload and the
 ratio, the gradient agreement of the two, the roofline of the dominant
-kernel (the multi-unit step), a served request stream (continuous
+kernel (resident steps: vector issue; the multi-unit step: HBM, timed beside
+the headline where that is not it), a served request stream (continuous
 batching; p50/p99 latency), ADVI/PSVI iterations on the device, the
 pseudo-spectral path, the CPU oracle timed on this host, and the
 CPU-runnable c0 case on CPU (one worker and a per-sample fan-out) and GPU.
@@ -42,6 +43,9 @@ sys.path.insert(0, REPO)
 
 METRIC = "misfit+grad samples/sec batched vs plain GPU @1e-4 grad tol; HBM GB/s frac; p50/p99"
 HBM_PEAK_GBS = 8000.0
+# one float operation a lane and cycle: 256 CUs x 64 lanes x 2.4 GHz (no packed
+# forms, no fused multiply-add: every operation rounds by itself)
+VALU_PEAK_TOPS = 39.3
 
 
 def log(msg):
@@ -93,6 +97,71 @@ def algorithmic_bytes_per_unit(p) -> int:
     sample."""
     nsave = math.ceil(p.nt / p.nt_interval)
     return p.nt * p.ntp * 32 + nsave * p.ni * 16 + p.nt * p.nr * 12
+
+
+def algorithmic_ops_per_unit(p) -> int:
+    """Separately rounded float operations of a (sample, shot) unit, forward
+    and adjoint: per padded point and step both axes' weighted sums and their
+    quotients and 2 p1 - p0 + (v dt)^2 lap, per stored inner point the second
+    time derivative and the imaging term (9).  Absorbing bands, source and
+    receivers are not counted."""
+    nsave = math.ceil(p.nt / p.nt_interval)
+    return 2 * p.nt * p.ntp * (2 * (3 * p.lc - 2) + 10) + nsave * p.ni * 9
+
+
+def resident_roofline(p, args, gpu_ms, plan) -> dict:
+    """Roofline entry of `args.steps` evaluations in `gpu_ms` with the fields
+    on the chip: the algorithm's float operations against the vector issue
+    rate (no HBM rate: the fields do not move).  A launch advances every unit
+    by up to plan["steps"] steps of one pass."""
+    from geopvi_amd.forward.fwi2d import solver
+    sch = solver.schedule(p, args.ckpt)
+    chunks = lambda n: -(-n // plan["steps"])  # noqa: E731
+    passes = [p.nt] + ([p.nt] if sch["nseg"] == 1 else
+                       2 * ([sch["ckpt"]] * (sch["nseg"] - 1) + [sch["last_len"]]))
+    launches = sum(chunks(n) for n in passes)
+    secs = gpu_ms * 1e-3 / args.steps
+    units = args.nsample * p.ns
+    achieved = units * algorithmic_ops_per_unit(p) / secs / 1e12
+    return {"bound": "valu", "achieved": round(achieved, 2), "peak": VALU_PEAK_TOPS, "unit": "Tops/s",
+            "frac": round(achieved / VALU_PEAK_TOPS, 4), "traffic": None, "kernel": "resident_kernel",
+            "launches_per_step": launches, "avg_launch_us": round(secs * 1e6 / launches, 1),
+            "dispatches_per_launch": 1, "slabs": plan["slabs"], "units_at_once": plan["clusters"],
+            "us_per_time_step": round(secs * 1e6 / sch["launches"], 3),
+            # what steps through memory would have to move in that time, not what moves
+            "step_launch_equivalent_GBs": round(units * algorithmic_bytes_per_unit(p) / secs / 1e9, 1)}
+
+
+def launch_roofline(p, args, eval_ms, variant, tb, lanes) -> dict:
+    """Roofline entry of an evaluation in `eval_ms` with every step a launch
+    through memory (multi-unit step kernel).  A launch here is one macro step
+    of every unit: `lanes` concurrent dispatches, each over its share of the
+    units, on the lanes' streams.  Algorithmic bytes of one launch / its
+    average time, the evaluation's time (events on the caller's stream, which
+    joins the lanes' streams at the end) over the launch count.  The step
+    launches are all but a few small set-up and reduction kernels, so this
+    bounds the step's average time from above; the profile under profiles/
+    gives the dispatches' union per launch from the kernel trace."""
+    from geopvi_amd.forward.fwi2d import solver
+    launches = solver.schedule(p, args.ckpt, tb)["launches"]
+    bytes_per_launch = args.nsample * p.ns * algorithmic_bytes_per_unit(p) / launches
+    avg_launch_s = eval_ms * 1e-3 / launches
+    achieved = bytes_per_launch / avg_launch_s / 1e9
+    traffic = profile = None
+    tj = _recorded_traffic()
+    if (tj and tj.get("tb") == tb and tj.get("variant") == variant and tj.get("ckpt") == args.ckpt
+            and tj.get("lanes", 1) == lanes):
+        traffic = tj.get("hbm_bytes_per_launch")
+        # the profile on record: the union of the lanes' dispatch intervals per
+        # launch (comparable with avg_launch_us) and one dispatch's average
+        profile = {"union_us_per_launch": tj.get("union_us_per_launch"),
+                   "avg_dispatch_us": tj.get("avg_dispatch_us"),
+                   "file": "profiles/step_multi_kernel_c1_16x20.md"}
+    return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "kernel": "step_multi_kernel",
+            "bytes_per_launch": int(bytes_per_launch), "launches_per_step": launches,
+            "avg_launch_us": round(avg_launch_s * 1e6, 3), "dispatches_per_launch": lanes,
+            **({"profile_on_record": profile} if profile else {})}
 
 
 def stream_3r1w_gbs(dev, mib: int = 512, reps: int = 10) -> float:
@@ -181,7 +250,7 @@ def serve_stream(args, rate, nreq, seed, dev, mix="bench", compare_batches=False
             solver.fwi_batch(p, vel, obs)
         torch.cuda.synchronize()
         tb = time.perf_counter() - t_b
-        batches = {"achieved_GBs": round(total_bytes / tb / 1e9, 1), "seconds": round(tb, 3),
+        batches = {"algorithmic_GBs": round(total_bytes / tb / 1e9, 1), "seconds": round(tb, 3),
                    "samples_per_s": round(total_samples / tb, 3)}
     policy = server_kw.get("store_policy", "auto")
     return {"requests": nreq, "rate_req_s": rate, "store": f"{policy}: {n_full} full store, {nreq - n_full} checkpointed",
@@ -193,7 +262,7 @@ def serve_stream(args, rate, nreq, seed, dev, mix="bench", compare_batches=False
             "admission_wait_p50_ms": round(float(np.percentile(wait, 50)) * 1e3, 1),
             "makespan_s": round(span, 3),
             "samples_per_s": round(total_samples / span, 3),
-            "achieved_GBs": round(total_bytes / span / 1e9, 1),
+            "algorithmic_GBs": round(total_bytes / span / 1e9, 1),
             **({"same_jobs_as_batches": batches} if batches else {})}
 
 
@@ -528,35 +597,12 @@ def main():
     ms_per_step = wall * 1e3 / args.steps
     value = args.nsample * args.steps / wall
 
-    # Roofline of the dominant kernel (multi-unit step, or with the automatic
-    # launch shape, variant -1, the resident steps: fields on the chip, a
-    # "launch" then being one step of every unit and the bytes those a step
-    # through memory would move).  A launch here is
-    # one macro step of every unit: `lanes` concurrent dispatches, each over
-    # its share of the units, on the lanes' streams.  Algorithmic bytes of
-    # one launch / its average time, the timed region's time (events on the
-    # caller's stream, which joins the lanes' streams at the end of every
-    # evaluation) over the launch count.  The step launches are all but a
-    # few small set-up and reduction kernels of the region, so this bounds
-    # the step's average time from above; the profile under profiles/ gives
-    # the dispatches' union per launch from the kernel trace.
-    sch = solver.schedule(p, args.ckpt, tb)
-    units = args.nsample * p.ns
-    launches = sch["launches"]
-    bytes_per_launch = units * algorithmic_bytes_per_unit(p) / launches
-    avg_launch_s = gpu_ms * 1e-3 / (args.steps * launches)
-    achieved = bytes_per_launch / avg_launch_s / 1e9
-    traffic = None
-    tj = _recorded_traffic()
-    profile = None
-    if (tj and tj.get("tb") == tb and tj.get("variant") == variant and tj.get("ckpt") == args.ckpt
-            and tj.get("lanes", 1) == lanes):
-        traffic = tj.get("hbm_bytes_per_launch")
-        # the profile on record: the union of the lanes' dispatch intervals per
-        # launch (comparable with avg_launch_us) and one dispatch's average
-        profile = {"union_us_per_launch": tj.get("union_us_per_launch"),
-                   "avg_dispatch_us": tj.get("avg_dispatch_us"),
-                   "file": "profiles/step_multi_kernel_c1_16x20.md"}
+    plan = solver.resident_plan(p, args.nsample, dev)
+    if plan:
+        lanes = 1   # the units are not split over streams
+    roofline = (resident_roofline(p, args, gpu_ms, plan) if plan else
+                launch_roofline(p, args, gpu_ms / args.steps, variant, tb, lanes))
+    us_per_step = gpu_ms * 1e3 / (args.steps * solver.schedule(p, args.ckpt, tb)["launches"])
 
     out = {
         "metric": METRIC,
@@ -576,23 +622,38 @@ def main():
                    "nsample": args.nsample, "shots": p.ns, "nt": p.nt, "grid": [p.nz, p.nx],
                    "ckpt_interval": args.ckpt, "tile_variant": variant, "launch_grid": grid,
                    "steps_per_launch": tb, "graph_steps": graph_steps, "lanes": lanes},
-        "roofline": {"bound": "hbm" if variant >= 0 else "valu", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "step_multi_kernel" if variant >= 0 else "resident_kernel", "bytes_per_launch": int(bytes_per_launch),
-                     "launches_per_step": launches, "avg_launch_us": round(avg_launch_s * 1e6, 3),
-                     "dispatches_per_launch": lanes, **({"profile_on_record": profile} if profile else {})},
+        "roofline": roofline,
     }
     if tune is not None:
         out["autotune"] = {"schedule": "forward with store + adjoint with imaging, 64 steps",
                            "chosen": tune.get("applied", f"{tune['variant']},{tune['grid']},{tune['tb']}"),
                            "us_per_time_step": tune["us_per_step"], "candidates": len(tune["timings"]),
-                           "us_per_launch_full_evaluation": round(avg_launch_s * 1e6, 3)}
-    del ws
+                           "us_per_time_step_full_evaluation": round(us_per_step, 3)}
     # What a plain streaming kernel with the step's read:write mix reaches on
     # this GPU (torch's addcmul: 3 reads, 1 write), for scale.
     stream = stream_3r1w_gbs(dev)
-    out["roofline"]["stream_3r1w_GBs"] = round(stream, 1)
-    out["roofline"]["frac_of_stream"] = round(achieved / stream, 4)
+    launches = roofline
+    if plan:
+        # The same batch with every step a launch through memory: what the HBM
+        # rate is measured on where the headline keeps its fields on the chip.
+        rec = _recorded_traffic() or {"variant": 4, "grid": 0, "tb": 1}
+        _lib.set_tuning(rec["variant"], rec["grid"], graph_steps)
+        _lib.set_time_blocking(rec["tb"])
+        run_batch()
+        ev0.record()
+        run_batch()
+        ev1.record()
+        torch.cuda.synchronize()
+        ms = ev0.elapsed_time(ev1)
+        _lib.set_tuning(variant, grid, graph_steps)
+        _lib.set_time_blocking(tb)
+        lanes_l = min(_lib.get_lanes(), max(2, args.nsample))
+        launches = launch_roofline(p, args, ms, rec["variant"], rec["tb"], lanes_l)
+        out["step_launches"] = {"samples_per_s": round(args.nsample * 1e3 / ms, 4), "roofline": launches}
+        log(f"step launches: {ms:.1f} ms an evaluation")
+    launches["stream_3r1w_GBs"] = round(stream, 1)
+    launches["frac_of_stream"] = round(launches["achieved"] / stream, 4)
+    del ws
 
     if not args.no_plain:
         vs0 = vel[0].contiguous()
