@@ -364,8 +364,10 @@ double step_launch_us(int lc, double points)
 {
     return kStepUs + kStepUsPerMpoint * (1 + kStepUsPerLc * (lc - 4)) * 1e-6 * points;
 }
-// Hardware queues whose launches may run at once (the runtime's default is 4
-// per process; 8 leaves room for a second process).
+// Hardware queues whose launches may run at once, as far as this process is
+// asked to keep to (the Python package asks for 8, the runtime's own default is
+// 4).  Streams of other priorities, with a CU mask or of other processes come
+// on top; where clusters then lack CUs they give up in time.
 int res_queues()
 {
     static const int queues = [] {

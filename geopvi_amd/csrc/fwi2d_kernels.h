@@ -61,7 +61,7 @@ hipError_t launch_advance(hipStream_t st, StepCtl* ctl, int n);
 hipError_t launch_ctl_set(hipStream_t st, StepCtl* ctl, int step, const int* ntiles4, const int* off4);
 hipError_t launch_zero(hipStream_t st, float* p, int64_t n);
 hipError_t launch_pad_velocity(hipStream_t st, const float* vin, float* vpad, int nx, int nz, int pml,
-                               int ntx, int ntz, int pitch, int64_t fe, int nsample);
+                               int ntx, int ntz, int pitch, int64_t stride, int nsample);
 hipError_t launch_tables(hipStream_t st, float* wav, int nt, float dt, float f0, float* wtab, int pml0);
 hipError_t launch_build_units(hipStream_t st, const JobDesc& j, UnitDesc* units, TileRef* tiles);
 hipError_t launch_grad_reduce(hipStream_t st, const float* gpriv, int64_t grad_stride, float* out, int ns,

@@ -395,12 +395,12 @@ hipError_t launch_zero(hipStream_t st, float* p, int64_t n)
 }
 
 hipError_t launch_pad_velocity(hipStream_t st, const float* vin, float* vpad, int nx, int nz, int pml,
-                               int ntx, int ntz, int pitch, int64_t fe, int nsample)
+                               int ntx, int ntz, int pitch, int64_t stride, int nsample)
 {
     const int64_t total = (int64_t)ntz * pitch * nsample;
     const int grid = (int)std::min<int64_t>((total + 255) / 256, 65536);
     hipLaunchKernelGGL(pad_velocity_kernel, dim3(grid), dim3(256), 0, st, vin, vpad, nx, nz, pml, ntx, ntz,
-                       pitch, fe, nsample);
+                       pitch, stride, nsample);
     return hipGetLastError();
 }
 

@@ -30,9 +30,12 @@
 //
 // What bounds it: vector issue, and per step about 2 us of exchange (a word
 // takes 0.7 us to a workgroup of the same XCD and up to 1.2 us across), barrier
-// and bookkeeping.  A point costs 80 vector instructions a 64-point row where
-// the update itself needs 54.  Memory is touched by the wavefield store, the
-// gradient and the halo only.  One 1024-thread workgroup per CU, as the two
+// and bookkeeping.  A 64-point row costs 83 vector instructions forward and 90
+// adjoint on average (320 units of 228x428, Lc 3, counters) where an interior
+// row's own block has 39 (157 for four rows); the bands, the bookkeeping of 16
+// wavefronts and the exchange are the rest.  They fill 83 and 79 % of the issue
+// slots.  Memory is touched by the wavefield store, the gradient and the halo
+// only.  One 1024-thread workgroup per CU, as the two
 // fields of a slab fill most of its LDS.  Microseconds a step of forward +
 // adjoint runs, one launch per step -> resident: 2 units of 52x68 padded points
 // 12.7 -> 4.7, 64 of 148x228 16.2 -> 7.4, 20 of 228x428 15.3 -> 8.1, 320 of
@@ -602,6 +605,11 @@ __device__ __forceinline__ bool res_strip(const ResUnit& k, const ResStep& s, Ld
     return asked;
 }
 
+// Points of a lane that a side block takes per round (64 units of 148x228 in
+// 1000 + 1000 steps take 14.70 ms with one, 15.39 with two; 320 of 228x428 171.1
+// and 175.6).
+constexpr int kResSideBlock = 1;
+
 // A side block, w columns wide: the item's points in row-major order (columns
 // counted inward from the edge), 64 at a time, kResSideBlock of these per
 // round, so that every lane has a point whatever the width.  ZB: the rows lie
@@ -611,7 +619,7 @@ template <int LC, bool ADJ, bool ZB>
 __device__ __forceinline__ void res_side(const ResUnit& k, const ResStep& s, LdsF* f1, LdsF* f0, int side, int lanepos,
                                          int w, int start, int dz, int cnt, int e0, bool hold, ResHeld& held)
 {
-    constexpr int B = 1;
+    constexpr int B = kResSideBlock;
     const int P = k.P, pml = k.pml, dP = dz * P;
     const int dx = side ? -1 : 1;
     const int rows64 = 64 / w, cols64 = 64 - rows64 * w;   // 64 points further on

@@ -87,12 +87,13 @@ constexpr int kLdsCx = 4096;         // LDS budget of one workgroup, in Cx (64 K
 // (2, 2); 134.7 with (4, 8) and 512 threads, 129.8 with (1, 2), 131.0 with
 // (1, 4) and 143.2 with (2, 4) and 128 threads.
 //
-// What bounds the passes: vector issue (about half of the cycles, 360 and 260
-// instructions a complex element and step in the row and column kernels) and
-// the latency of 6 to 8 LDS round trips with a barrier each, at 5 wavefronts a
-// SIMD (the two LDS buffers).  Of the instructions a quarter is double
-// arithmetic, the rest index splits and addresses, so those come from the
-// host or from scalar loads: 148 us a step before, 114 us since.
+// What bounds the passes: vector issue (two thirds of the slots with two lanes'
+// kernels at once, 44 and 31 % in the row and the column kernel alone; 496 and
+// 286 instructions a complex element and step, counters) and the latency of 6
+// to 8 LDS round trips with a barrier each, at 5 wavefronts a SIMD (the two LDS
+// buffers).  Of the instructions 28 and 47 % are double arithmetic, a third
+// index splits and addresses even though these come from the host or from
+// scalar loads where they can: 148 us a step before, 114 us since.
 constexpr int kMaxPairs = 2;
 constexpr int kMaxCols = 4;
 
