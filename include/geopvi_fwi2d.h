@@ -126,8 +126,8 @@ int gpvi_fwi2d_batch(const gpvi_fwi2d_params *p, int nsample, const float *vel_i
 
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
- * forbid hipMalloc).  gpvi_fwi2d_batch with GPVI_PHASE_ALL and one launch
- * per step, its workspace taken from a fixed device array of
+ * forbid hipMalloc).  gpvi_fwi2d_batch with GPVI_PHASE_ALL (one launch per
+ * step where the fields do not stay on the chip), its workspace taken from a fixed device array of
  * GPVI_STATIC_SCRATCH_BYTES per GPU (held from library load until the
  * process ends) instead of an argument: the caller passes inputs and outputs
  * only.  Nothing is allocated.  A job whose workspace
