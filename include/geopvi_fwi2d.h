@@ -102,8 +102,9 @@ int gpvi_fwi2d_forward_device(const gpvi_fwi2d_params *p, const float *vel_inner
 
 /* ---- Batched solver: nsample samples x ns shots per launch ----
  * Replaces the per-sample process fan-out around fwi_2D
- * (geopvi/forward/fwi2d/posterior.py:131-149) with one launch per time step
- * over every (sample, shot) unit, replayed as HIP graph segments.
+ * (geopvi/forward/fwi2d/posterior.py:131-149) with launches over every
+ * (sample, shot) unit: up to 256 time steps each with the fields on the chip
+ * where that is faster, else one per time step, replayed as HIP graph segments.
  *   vel_inner  [nsample][nz][nx]   record_obs [ns][nt][nr] (shared)
  *   record_syn [nsample][ns][nt][nr]   grad [nsample][nz][nx] (+=)
  *   misfit     [nsample] double, 0.5*sum((syn-obs)^2) (posterior.py:109)
@@ -183,8 +184,8 @@ int gpvi_fwi2d_get_time_blocking(void);
  * events.  The step launches of one group then fill the GPU while those of
  * another drain.  Streams only overlap on hardware queues of their own
  * (GPU_MAX_HW_QUEUES).  Results are the same bits for every n.
- * Process-wide; one lane is always used with GPVI_FLAG_ONE_STREAM, for a
- * single unit and by gpvi_fwi2d_batch_static. */
+ * Process-wide; one lane is always used with the fields on the chip, with
+ * GPVI_FLAG_ONE_STREAM, for a single unit and by gpvi_fwi2d_batch_static. */
 int gpvi_fwi2d_set_lanes(int lanes);
 int gpvi_fwi2d_get_lanes(void);
 
